@@ -12,6 +12,9 @@ namespace hbr {
 // Rows per partition tile (one workgroup).
 constexpr uint32_t kPartTile = 2048;
 constexpr uint32_t kPartThreads = 256;
+// Rows a thread of the one-pass partition (hbr_part_move) holds: a tile is
+// this many per thread of its workgroup.
+constexpr uint32_t kMoveRows = 8;
 // Histogram workgroups: threads, and the fewest rows a tile is cut to (tiles
 // are sized per launch so that about one wave of workgroups covers it).
 constexpr uint32_t kHistThreads = 512;
@@ -264,10 +267,12 @@ struct PartSplit {
     uint32_t pad[3];
 };
 
-// Device decision per split after the scan of tile counts.
-struct PartOut {
+// A split's children after the partition: their row counts, the smaller
+// child (the left one when equal) being the built one. hbr_part_move takes
+// each tile's runs of both with one 64-bit atomic add.
+struct alignas(8) PartOut {
     uint32_t left_len;
-    uint32_t built_left;    // 1: the left child is the smaller (built) one
+    uint32_t right_len;
     uint32_t pad[2];
 };
 
@@ -295,6 +300,8 @@ struct PartArgs {
     uint32_t csr_ascending;      // every CSR row's global bins ascend: routing binary-searches them
     uint32_t pad;
     const uint32_t *cat_tables;  // kCatWords words per categorical split: its left local bins
+    uint32_t move_tile;          // hbr_part_move: rows per tile (kMoveRows x its threads)
+    uint32_t pad2;
 };
 
 // ---- histograms ----------------------------------------------------------------
@@ -713,6 +720,9 @@ struct GrowArgs {
     uint32_t n_trees;
     uint32_t tree_bytes;
     uint32_t *tree_nodes;
+    PartOut *out;                 // this level's splits' partition results, cleared for hbr_part_move
+    uint32_t part_tile;           // rows of a partition tile
+    uint32_t pad;
 };
 
 // Most slots a device-grown tree may hold (the LDS free-slot table).

@@ -1473,6 +1473,16 @@ PartArgs Engine::part_args() const {
     return a;
 }
 
+// Threads of the one-pass partition's workgroups: small tiles fill the chip
+// on small levels, large ones queue less on a split's word (about 14 ns a
+// tile). Measured us per level, 256 / 512 / 1,024 threads: 100k rows 7.1 /
+// 7.8 / 8.3; 1M rows 10.7 / 10.0 / 10.4; 10.5M rows 68 / 48 / 40; ten trees
+// of 2M rows 98 / 71 / 65 (count, scan and scatter passes in their place:
+// 12.2, 16.4, 42.6 and 73.6).
+uint32_t Engine::part_move_threads(uint64_t rows) const {
+    return rows <= (1u << 19) ? 256u : rows <= (1u << 21) ? 512u : 1024u;
+}
+
 std::vector<LevelChild> Engine::level(const std::vector<LevelSplit> &splits, bool terminal) {
     const uint32_t P = (uint32_t)splits.size();
     std::vector<LevelChild> children(2 * P);
@@ -1586,7 +1596,7 @@ std::vector<LevelChild> Engine::level(const std::vector<LevelSplit> &splits, boo
         R.seg = Segment{pseg.offset + nl, pseg.len - nl, pseg.buf ^ 1u};
         counters.partition_rows += pseg.len;
         if (!terminal) {
-            const bool built_left = po[i].built_left != 0;
+            const bool built_left = po[i].left_len <= po[i].right_len;
             L.slot = built_left ? fresh[i] : splits[i].parent_slot;
             R.slot = built_left ? splits[i].parent_slot : fresh[i];
             L.best = best_staged[2 * i];
@@ -1757,7 +1767,9 @@ Engine::TreeTicket Engine::queue_device_forest(uint32_t n_trees, uint64_t max_de
     if (!reserve_slots(slot_cap)) fail(kRefused, "histogram slots do not fit in device memory");
     const uint32_t pmax_all = n_trees * (depth >= 2 ? 1u << (depth - 2) : 1u);
     // every level partitions at most n_trees x n_rows rows, each tree's in its own region
-    const uint32_t row_tiles = (uint32_t)ceil_div((uint64_t)n_trees * n_rows_, kPartTile);
+    const uint32_t move_threads = part_move_threads((uint64_t)n_trees * n_rows_);
+    const uint32_t move_tile = move_threads * kMoveRows;
+    const uint32_t row_tiles = (uint32_t)ceil_div((uint64_t)n_trees * n_rows_, move_tile);
     for (int b = 0; b < 2; b++) {
         g_front_[b].reserve(std::max<uint32_t>(slot_cap, n_trees));
         g_splits_[b].reserve(pmax_all);
@@ -1767,8 +1779,6 @@ Engine::TreeTicket Engine::queue_device_forest(uint32_t n_trees, uint64_t max_de
     d_hnodes_.reserve(pmax_all);
     d_snodes_.reserve(2 * pmax_all);
     d_best_.reserve(std::max<uint32_t>(2 * pmax_all, n_trees));
-    d_tile_left_.reserve(row_tiles + pmax_all);
-    d_decisions_.reserve((size_t)(row_tiles + pmax_all) * (kPartTile / 64));
     d_tile_split_.reserve(row_tiles + pmax_all);
     d_tree_nodes_.reserve(n_trees);
     GrowCounts *counts = grow_counts_dev();
@@ -1838,6 +1848,8 @@ Engine::TreeTicket Engine::queue_device_forest(uint32_t n_trees, uint64_t max_de
         g.n_trees = n_trees;
         g.tree_bytes = (uint32_t)stride;
         g.tree_nodes = d_tree_nodes_.get();
+        g.out = g_pout_[lv & 1].get();
+        g.part_tile = move_tile;
         dev_.launch(n_trees == 1 ? "hbr_grow_decide" : "hbr_grow_decide_batch", dim3(1), dim3(512), g);
         if (terminal) break;
         PartArgs a = part_args();
@@ -1847,9 +1859,8 @@ Engine::TreeTicket Engine::queue_device_forest(uint32_t n_trees, uint64_t max_de
         a.out = g_pout_[lv & 1].get();
         a.grow = counts;
         a.tile_split = d_tile_split_.get();
-        dev_.launch("hbr_part_count", dim3(a.n_tiles), dim3(kPartThreads), a);
-        dev_.launch("hbr_part_scan", dim3(pmax), dim3(1024), a);
-        dev_.launch("hbr_part_scatter", dim3(a.n_tiles), dim3(kPartThreads), a);
+        a.move_tile = move_tile;
+        dev_.launch("hbr_part_move", dim3(a.n_tiles), dim3(move_threads), a);
         launch_hist(d_hnodes_.get(), pmax, nullptr, a.splits, a.out, nullptr, counts);
         launch_scan(d_snodes_.get(), 2 * pmax, a.splits, a.out, d_best_.get(), counts);
     }

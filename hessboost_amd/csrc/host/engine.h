@@ -409,6 +409,7 @@ private:
     DBuf<uint32_t> poison_;
     std::vector<int8_t> monotone_host_;
     PartArgs part_args() const;
+    uint32_t part_move_threads(uint64_t rows) const;
     void scan_host_nodes(const std::vector<ScanNode> &nodes, ScanBest *out, uint32_t *sets = nullptr);
     void launch_gradients(const hbr_device_loss &loss, uint32_t output);
     GradArgs grad_args(const hbr_device_loss &loss);

@@ -153,7 +153,7 @@ __device__ __forceinline__ void grow_decide(const GrowArgs &a) {
             seg.buf = sp.seg.buf ^ 1u;
             seg.offset = c == 0 ? sp.seg.offset : sp.seg.offset + nl;
             seg.len = c == 0 ? nl : sp.seg.len - nl;
-            const bool built = (c == 0) == (po.built_left != 0);
+            const bool built = (c == 0) == (po.left_len <= po.right_len);
             slot = built ? sp.fresh_slot : sp.parent_slot;
             total = g.total;
             lower = g.lower;
@@ -162,7 +162,7 @@ __device__ __forceinline__ void grow_decide(const GrowArgs &a) {
             tree = g.tree;
             if (c == 0) {
                 part_rows += sp.seg.len;
-                hist_rows += po.built_left ? nl : sp.seg.len - nl;
+                hist_rows += min(po.left_len, po.right_len);
             }
         }
         if (active && (b.flags & kScanNearTie)) near_ties++;
@@ -201,7 +201,7 @@ __device__ __forceinline__ void grow_decide(const GrowArgs &a) {
                         rh >= a.reg.min_child_weight;
             }
         }
-        const uint32_t tiles = valid && !a.terminal ? (seg.len + kPartTile - 1) / kPartTile : 0u;
+        const uint32_t tiles = valid && !a.terminal ? (seg.len + a.part_tile - 1) / a.part_tile : 0u;
         uint32_t n_valid, n_tiles;
         const uint32_t i = split_carry + block_exclusive_scan<kGrowThreads>(valid ? 1u : 0u, &n_valid);
         const uint32_t tile_begin = tile_carry + block_exclusive_scan<kGrowThreads>(tiles, &n_tiles);
@@ -293,6 +293,7 @@ __device__ __forceinline__ void grow_decide(const GrowArgs &a) {
                 p.parent_slot = slot;
                 p.tree = tree;
                 a.splits[i] = p;
+                a.out[i] = PartOut{};
                 s_tile_begin[i] = tile_begin;
                 HistNode h{};
                 h.from_split = 1;

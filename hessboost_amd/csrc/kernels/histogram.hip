@@ -26,7 +26,7 @@ __device__ __forceinline__ Seg resolve_node(const PlanArgs &a, const HistNode &n
     Seg s;
     s.buf = sp.seg.buf ^ 1u;
     s.pad = 0;
-    if (po.built_left) {
+    if (po.left_len <= po.right_len) {
         s.offset = sp.seg.offset;
         s.len = po.left_len;
     } else {

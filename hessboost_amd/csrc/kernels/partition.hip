@@ -190,7 +190,7 @@ extern "C" __global__ __launch_bounds__(1024) void hbr_part_scan(PartArgs a) {
     if (threadIdx.x == 0) {
         PartOut o;
         o.left_len = carry;
-        o.built_left = carry <= sp.seg.len - carry ? 1u : 0u;
+        o.right_len = sp.seg.len - carry;
         o.pad[0] = o.pad[1] = 0;
         a.out[s] = o;
     }
@@ -251,6 +251,98 @@ extern "C" __global__ __launch_bounds__(256) void hbr_part_scatter(PartArgs a) {
             dst[left_len + right_before + rights] = r[k];
         }
     }
+}
+
+// The partition of a device-grown level in one pass. Its children's rows
+// may stand in any order (every sum over them is an integer sum, and the
+// margins are walked in row order), so a tile needs no scan of the tiles
+// before it: its workgroup routes kMoveRows rows a thread, takes a run of
+// the left child's rows (from the segment's start) and one of the right
+// child's (from its end) with one 64-bit atomic add to the split's PartOut,
+// and writes both runs in the tile's row order. The ids are read and
+// written once; the routing bytes are gathered (a 128-byte line for a few
+// rows at deep levels), and the tiles of one split queue on its word at
+// about 14 ns each.
+template <typename Bin, bool MISSING>
+__device__ __forceinline__ void part_move(const PartArgs &a, const Bin *cols) {
+    __shared__ uint32_t s_left[1024 / kWave], s_rows[1024 / kWave];
+    __shared__ uint32_t s_base[2];
+    const uint32_t tile = blockIdx.x;
+    const uint32_t s = a.tile_split[tile];  // loaded with the tile count (the table covers the grid)
+    if (tile >= a.grow->n_tiles) return;    // uniform across the workgroup
+    const PartSplit sp = a.splits[s];
+    const uint32_t wave = threadIdx.x / kWave, waves = blockDim.x / kWave, lane = lane_id();
+    const uint32_t *src = a.src_rows[sp.seg.buf] + sp.seg.offset;
+    const uint32_t id0 = sp.identity ? sp.seg.offset % a.n_rows : 0u;
+    // a wave owns kMoveRows x 64 consecutive rows of the tile
+    const uint32_t base = (tile - sp.tile_begin) * a.move_tile + wave * (kMoveRows * kWave);
+    uint32_t r[kMoveRows];
+#pragma unroll
+    for (uint32_t k = 0; k < kMoveRows; k++) {
+        const uint32_t j = base + k * kWave + lane;
+        r[k] = j < sp.seg.len ? (sp.identity ? id0 + j : src[j]) : 0xffffffffu;
+    }
+    const Bin *col = cols + (size_t)sp.feature * a.n_rows;
+    uint32_t b[kMoveRows];
+#pragma unroll
+    for (uint32_t k = 0; k < kMoveRows; k++) b[k] = r[k] != 0xffffffffu ? (uint32_t)col[r[k]] : 0xffffffffu;
+    if constexpr (MISSING) {  // a missing cell's bin takes the default way's side of the limit
+        const uint64_t *bits = a.missing + (size_t)sp.feature * a.words;
+        uint64_t w[kMoveRows];
+#pragma unroll
+        for (uint32_t k = 0; k < kMoveRows; k++) w[k] = r[k] != 0xffffffffu ? bits[r[k] >> 6] : 0ull;
+#pragma unroll
+        for (uint32_t k = 0; k < kMoveRows; k++)
+            if ((w[k] >> (r[k] & 63u)) & 1ull) b[k] = 0xfffffffeu;
+    }
+    uint64_t m[kMoveRows];
+    uint32_t lefts = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kMoveRows; k++) {
+        const bool left = MISSING && b[k] == 0xfffffffeu ? sp.default_left != 0 : b[k] < sp.limit;
+        m[k] = __ballot(left && r[k] != 0xffffffffu);
+        lefts += (uint32_t)__popcll(m[k]);
+    }
+    const uint32_t mine = base < sp.seg.len ? min(sp.seg.len - base, kMoveRows * (uint32_t)kWave) : 0u;
+    if (lane == 0) {
+        s_left[wave] = lefts;
+        s_rows[wave] = mine;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t left = 0, rows = 0;
+        for (uint32_t w = 0; w < waves; w++) {
+            left += s_left[w];
+            rows += s_rows[w];
+        }
+        const unsigned long long take = (unsigned long long)left | ((unsigned long long)(rows - left) << 32);
+        const unsigned long long at = atomicAdd(reinterpret_cast<unsigned long long *>(&a.out[s].left_len), take);
+        s_base[0] = (uint32_t)at;
+        s_base[1] = sp.seg.len - (uint32_t)(at >> 32) - (rows - left);
+    }
+    __syncthreads();
+    uint32_t *dst = a.dst_rows[sp.seg.buf ^ 1u] + sp.seg.offset;
+    uint32_t lo = s_base[0], hi = s_base[1];
+    for (uint32_t w = 0; w < wave; w++) {
+        lo += s_left[w];
+        hi += s_rows[w] - s_left[w];
+    }
+    const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+    for (uint32_t k = 0; k < kMoveRows; k++) {
+        const bool some = r[k] != 0xffffffffu;  // the rows of a wave's 64 that exist come first
+        const uint64_t all = __ballot(some);
+        const uint32_t left_before = (uint32_t)__popcll(m[k] & below);
+        if (some) dst[(m[k] >> lane) & 1ull ? lo + left_before : hi + (lane - left_before)] = r[k];
+        const uint32_t n_left = (uint32_t)__popcll(m[k]);
+        lo += n_left;
+        hi += (uint32_t)__popcll(all) - n_left;
+    }
+}
+
+extern "C" __global__ __launch_bounds__(1024, 8) void hbr_part_move(PartArgs a) {
+    if (a.missing) part_move<uint8_t, true>(a, a.cols8);
+    else part_move<uint8_t, false>(a, a.cols8);
 }
 
 // Leaf values onto the margins of each leaf's rows (training/margins.rs:247-289,

@@ -226,8 +226,8 @@ __device__ __forceinline__ uint32_t scan_nodes(const ScanArgs &a) { return a.gro
 __device__ __forceinline__ uint32_t node_slot(const ScanArgs &a, const ScanNode &nd) {
     if (!nd.from_split) return nd.slot;
     const PartSplit sp = a.splits[nd.split];
-    const uint32_t built_left = a.part_out[nd.split].built_left;
-    const bool built = nd.child == 0 ? built_left != 0 : built_left == 0;
+    const PartOut po = a.part_out[nd.split];
+    const bool built = (nd.child == 0) == (po.left_len <= po.right_len);
     return built ? sp.fresh_slot : sp.parent_slot;
 }
 
@@ -242,8 +242,8 @@ using namespace hbr;
 // A node's row count: its record's, or the partition's for a child of a split.
 __device__ __forceinline__ uint32_t node_rows(const ScanArgs &a, const ScanNode &nd) {
     if (!nd.from_split) return nd.rows;
-    const uint32_t left = a.part_out[nd.split].left_len;
-    return nd.child == 0 ? left : a.splits[nd.split].seg.len - left;
+    const PartOut po = a.part_out[nd.split];
+    return nd.child == 0 ? po.left_len : po.right_len;
 }
 
 // x rounded up to f32.

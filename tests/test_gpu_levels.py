@@ -1,0 +1,65 @@
+"""The kernels of a device-grown level at the sizes where they can go wrong
+(edges of tiles, remainders, the smallest and largest of their ranges): trees
+and margins against growth decided by the host, level by level, whose
+kernels share none of them, bit for bit."""
+import numpy as np
+import pytest
+
+import hessboost_amd as hb
+
+pytestmark = pytest.mark.gpu
+
+
+def _fit(x, y, params, rounds, weight=None):
+    engine = hb.DMatrix(x, label=y).engine(params.get("max_bin", 256))
+    t = hb.Trainer(engine, params, y, weight)
+    engine.set_profiling(True)
+    t.boost(rounds)
+    launches = {k: v["calls"] for k, v in engine.kernel_stats().items()}
+    engine.set_profiling(False)
+    return t.trees(), t.margins(), launches
+
+
+def _same(a, b):
+    (ta, ma, _), (tb, mb, _) = a, b
+    assert len(ta) == len(tb)
+    for i, (p, q) in enumerate(zip(ta, tb)):
+        for key in p:
+            assert np.array_equal(p[key], q[key]), (i, key)
+    assert np.array_equal(ma.view(np.uint32), mb.view(np.uint32))
+
+
+def _data(n, f, nan, seed, classes=0):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((n, f), dtype=np.float32)
+    s = x[:, 0] - 0.5 * x[:, 1 % f] * x[:, 2 % f]
+    if classes:
+        y = np.clip(np.floor(s * 0.7 + classes / 2), 0, classes - 1)
+    else:
+        y = s > 0
+    if nan:
+        x[rng.random(x.shape) < nan] = np.nan
+    return x, y.astype(np.float32)
+
+
+def _both(monkeypatch, x, y, params, rounds, weight=None):
+    device = _fit(x, y, params, rounds, weight)
+    monkeypatch.setenv("HBROCM_DEVICE_GROW", "0")
+    host = _fit(x, y, params, rounds, weight)
+    return device, host
+
+
+# tiles of 2,048, 4,096 and 8,192 rows (up to 2^19 and 2^21 rows, and beyond)
+@pytest.mark.parametrize("n,f,nan,classes", [
+    (1, 3, 0.0, 0), (63, 3, 0.0, 0), (2047, 5, 0.1, 0), (2048, 5, 0.0, 0), (2049, 33, 0.1, 0), (4097, 4, 0.0, 3),
+    (2**19 + 1, 4, 0.0, 0), (2**19 + 4095, 4, 0.1, 0), (2**21 + 8191, 3, 0.0, 0), (700_001, 3, 0.0, 3),
+])
+def test_one_pass_partition_gives_the_host_levels_trees(monkeypatch, n, f, nan, classes):
+    x, y = _data(n, f, nan, seed=n, classes=classes)
+    params = {"objective": "multi:softprob" if classes else "binary:logistic", "max_depth": 5, "eta": 0.3,
+              "base_score": 0.5}
+    if classes:
+        params["num_class"] = classes
+    device, host = _both(monkeypatch, x, y, params, 2)
+    assert device[2].get("hbr_part_move", 0) > 0 and "hbr_part_count" not in device[2]
+    _same(device, host)
