@@ -15,10 +15,11 @@ constexpr uint32_t kPartThreads = 256;
 // Rows a thread of the one-pass partition (hbr_part_move) holds: a tile is
 // this many per thread of its workgroup.
 constexpr uint32_t kMoveRows = 8;
-// Histogram workgroups: threads, and the fewest rows a tile is cut to (tiles
-// are sized per launch so that about one wave of workgroups covers it).
+// Histogram workgroups: threads, and the fewest rows a tile is ever cut to
+// (tiles are sized per launch so that about one wave of workgroups covers
+// it, unless its rows are few: PlanArgs::min_cost).
 constexpr uint32_t kHistThreads = 512;
-constexpr uint32_t kHistMinRows = 4096;
+constexpr uint32_t kHistMinRows = 256;
 // Bins of one feature the split scan processes per pass (4 per lane).
 constexpr uint32_t kScanChunk = 256;
 // Threads of the elementwise kernels.
@@ -334,7 +335,8 @@ struct HistNode {
 };
 
 // Device tiling of a histogram launch: each node's rows cut into tiles of
-// `tile_rows` rows (a multiple of 64, at least min_rows), the smallest size
+// `tile_rows` rows (a multiple of 64, at least kHistMinRows and
+// sqrt(min_cost x the launch's rows)), the smallest size
 // that gives at most target_tiles tiles (one tile per node when the nodes
 // outnumber it); never more than target_tiles + n_nodes tiles.
 struct PlanArgs {
@@ -345,7 +347,7 @@ struct PlanArgs {
     const PartOut *part_out;
     HistTile *tiles;
     uint32_t *counts;           // [0] tiles, [1] tile_rows
-    uint32_t min_rows;
+    uint32_t min_cost;          // a tile's fixed cost in rows' (Engine::tile_cost)
     uint32_t fuse_subtract;     // built children of splits also update their siblings (dense kernels)
     const GrowCounts *grow;     // non-null: one node per split of the level, n_splits read from here
 };

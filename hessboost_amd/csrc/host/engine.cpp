@@ -1228,6 +1228,16 @@ void Engine::set_scan_params(const ScanParams &p, const std::vector<int8_t> &mon
 
 // Histograms of a batch of nodes into their slots: the plan kernel cuts the
 // nodes' rows into tiles (about `per_cu` resident workgroups per CU over the
+// The fewest rows a tile is worth, as PlanArgs::min_cost: a tile's partials
+// are written and read back (about 64 ns a group of the launch, whose
+// workgroups share the memory), its rows take a workgroup about 5.9 ns each
+// (32 features' LDS atomics; 16 wide ones' half of that), so with R rows the
+// shortest launch has tiles of about sqrt(R x groups x 64 / 5.9) rows. A CSR
+// row costs its wave a chain of dependent loads, about 31 ns.
+uint32_t Engine::tile_cost(uint32_t groups) const {
+    return groups * (dense16_ ? 22u : dense_u8_ ? 11u : 2u);
+}
+
 // launch), then one workgroup per (tile, feature group). Dense u8 tiles
 // write their sums with plain stores (the reduce kernel adds up nodes of
 // several tiles); CSR tiles add into slots zeroed first.
@@ -1262,7 +1272,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     p.part_out = part_out_dev;
     p.tiles = d_htiles_.get();
     p.counts = d_hcounts_.get();
-    p.min_rows = kHistMinRows;
+    p.min_cost = tile_cost(groups);
     p.fuse_subtract = dense ? 1u : 0u;
     p.grow = grow;
     dev_.launch("hbr_hist_plan", dim3(1), dim3(256), p);
@@ -2411,7 +2421,7 @@ bool Engine::build_rows_fixed(const uint32_t *rows, uint64_t m, double *out, uin
     p.target_tiles = (uint32_t)target;
     p.tiles = tiles;
     p.counts = counts;
-    p.min_rows = kHistMinRows;
+    p.min_cost = tile_cost(groups);
     dev_.launch("hbr_hist_plan", dim3(1), dim3(256), p);
 
     HistArgs a{};

@@ -410,6 +410,7 @@ private:
     std::vector<int8_t> monotone_host_;
     PartArgs part_args() const;
     uint32_t part_move_threads(uint64_t rows) const;
+    uint32_t tile_cost(uint32_t groups) const;
     void scan_host_nodes(const std::vector<ScanNode> &nodes, ScanBest *out, uint32_t *sets = nullptr);
     void launch_gradients(const hbr_device_loss &loss, uint32_t output);
     GradArgs grad_args(const hbr_device_loss &loss);

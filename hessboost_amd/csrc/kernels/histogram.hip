@@ -315,8 +315,9 @@ extern "C" __global__ __launch_bounds__(256) void hbr_hist_plan(PlanArgs a) {
     // each counted against every node at once; the smallest that fits wins.
     // hi = the longest node fits whenever the nodes do not outnumber the
     // target (one tile each).
-    const unsigned long long lo =
-        max((total + a.target_tiles - 1) / a.target_tiles, (unsigned long long)a.min_rows);
+    const unsigned long long worth = (unsigned long long)__builtin_sqrtf((float)total * (float)a.min_cost);
+    const unsigned long long lo = max((total + a.target_tiles - 1) / a.target_tiles,
+                                      max(worth, (unsigned long long)kHistMinRows));
     const unsigned long long hi = max(longest, lo);
     const double ratio = (double)hi / (double)lo;
     unsigned long long cand = threadIdx.x == blockDim.x - 1

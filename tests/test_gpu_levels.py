@@ -15,7 +15,7 @@ def _fit(x, y, params, rounds, weight=None):
     t = hb.Trainer(engine, params, y, weight)
     engine.set_profiling(True)
     t.boost(rounds)
-    launches = {k: v["calls"] for k, v in engine.kernel_stats().items()}
+    launches = {k: v[1] for k, v in engine.kernel_stats().items()}
     engine.set_profiling(False)
     return t.trees(), t.margins(), launches
 
@@ -63,3 +63,24 @@ def test_one_pass_partition_gives_the_host_levels_trees(monkeypatch, n, f, nan, 
     device, host = _both(monkeypatch, x, y, params, 2)
     assert device[2].get("hbr_part_move", 0) > 0 and "hbr_part_count" not in device[2]
     _same(device, host)
+
+
+# few rows (one tile), about one tile's worth, one wave of tiles and beyond,
+# dense groups of 32 features (one and several), 16-bit bins and sparse rows
+@pytest.mark.parametrize("n", [1, 255, 257, 5_000, 60_001, 300_000])
+@pytest.mark.parametrize("f,bins,density", [(7, 256, 1.0), (40, 256, 1.0), (20, 400, 1.0), (60, 256, 0.1)])
+def test_histogram_tiles_sum_every_row(n, f, bins, density):
+    rng = np.random.default_rng(n + f)
+    x = rng.standard_normal((n, f), dtype=np.float32)
+    if density < 1.0:
+        x[rng.random(x.shape) >= density] = np.nan
+    engine = hb.DMatrix(x).engine(bins)
+    pairs = rng.integers(-8, 9, (n, 2)).astype(np.float32)  # every sum exact
+    engine.prepare(pairs)
+    hist = engine.build(np.arange(n))
+    index = hb.DMatrix(x).index(bins)
+    row_ptr, row_bins = index.row_bins()
+    rows = np.repeat(np.arange(n), np.diff(row_ptr.astype(np.int64)))
+    for c in (0, 1):
+        want = np.bincount(row_bins, weights=pairs[rows, c].astype(np.float64), minlength=len(hist))
+        assert np.array_equal(hist[:, c], want)
