@@ -13,6 +13,8 @@ namespace hbr {
 namespace {
 
 constexpr uint32_t kLeafTile = 4096;
+// Threads of the passes that end in a fold of maxima: few, large workgroups.
+constexpr uint32_t kFoldThreads = 1024;
 
 uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
@@ -786,10 +788,10 @@ void Engine::launch_gradients(const hbr_device_loss &loss, uint32_t output) {
     root_partials_ = 0;  // the staged pairs are no longer the walk's
     pair_array_stale_ = false;
     row_pairs_min_hess_ = loss.min_hess;
-    // grid-stride: a few workgroups per CU, one max fold each
-    const uint32_t grad_blocks = std::min<uint32_t>(std::max<uint32_t>(1, ceil_div(n_rows_, kThreads)),
-                                                    (uint32_t)dev_.cu_count() * 8);
-    dev_.launch("hbr_gradients", dim3(grad_blocks), dim3(kThreads), a);
+    // grid-stride: two workgroups per CU, one max fold each
+    const uint32_t grad_blocks = std::min<uint32_t>(std::max<uint32_t>(1, ceil_div(n_rows_, kFoldThreads)),
+                                                    (uint32_t)dev_.cu_count() * 2);
+    dev_.launch("hbr_gradients", dim3(grad_blocks), dim3(kFoldThreads), a);
 }
 
 // The exponents of the folded maxima, on the host (the device's rule), and
@@ -806,9 +808,9 @@ bool Engine::check_scale(QScale host, uint32_t bound_g_bits, uint32_t bound_h_bi
 bool Engine::compute_gradients(const hbr_device_loss &loss, uint32_t output) {
     launch_gradients(loss, output);
     {  // the grains of the pairs, for the exact-domain check of later sums
-        const uint32_t blocks = std::min<uint32_t>(std::max<uint32_t>(1, ceil_div(n_rows_, kThreads)),
-                                                   (uint32_t)dev_.cu_count() * 8);
-        dev_.launch("hbr_grain_fold", dim3(blocks), dim3(kThreads), grad_args(loss));
+        const uint32_t blocks = std::min<uint32_t>(std::max<uint32_t>(1, ceil_div(n_rows_, kFoldThreads)),
+                                                   (uint32_t)dev_.cu_count() * 2);
+        dev_.launch("hbr_grain_fold", dim3(blocks), dim3(kFoldThreads), grad_args(loss));
     }
     QScale *q = static_cast<QScale *>(stage_.alloc(sizeof(QScale)));
     HBR_HIP(hipMemcpyAsync(q, scale_dev(), sizeof(QScale), hipMemcpyDeviceToHost, dev_.stream()));
@@ -1226,8 +1228,6 @@ void Engine::set_scan_params(const ScanParams &p, const std::vector<int8_t> &mon
     }
 }
 
-// Histograms of a batch of nodes into their slots: the plan kernel cuts the
-// nodes' rows into tiles (about `per_cu` resident workgroups per CU over the
 // The fewest rows a tile is worth, as PlanArgs::min_cost: a tile's partials
 // are written and read back (about 64 ns a group of the launch, whose
 // workgroups share the memory), its rows take a workgroup about 5.9 ns each
@@ -1238,6 +1238,8 @@ uint32_t Engine::tile_cost(uint32_t groups) const {
     return groups * (dense16_ ? 22u : dense_u8_ ? 11u : 2u);
 }
 
+// Histograms of a batch of nodes into their slots: the plan kernel cuts the
+// nodes' rows into tiles (about `per_cu` resident workgroups per CU over the
 // launch), then one workgroup per (tile, feature group). Dense u8 tiles
 // write their sums with plain stores (the reduce kernel adds up nodes of
 // several tiles); CSR tiles add into slots zeroed first.
