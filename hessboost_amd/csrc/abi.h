@@ -209,6 +209,23 @@ struct SoftmaxArgs {
     float min_hess;
 };
 
+// A trainer's start. Margins [n / k][k] at base[k]; and how many labels equal
+// 0, 1, ..., k - 1 (k <= kSoftmaxMaxClasses; counts zeroed before).
+struct FillArgs {
+    float *margins;
+    const float *base;
+    uint64_t n;
+    uint32_t k;
+    uint32_t pad;
+};
+struct LabelArgs {
+    const float *labels;
+    unsigned long long *counts;
+    uint64_t n;
+    uint32_t k;
+    uint32_t pad;
+};
+
 // ---- row buffers -------------------------------------------------------------
 struct IotaArgs {
     uint32_t *rows;

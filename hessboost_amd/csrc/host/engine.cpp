@@ -465,8 +465,8 @@ void Engine::read_index(uint8_t *rows8, uint8_t *cols8, uint64_t *missing, uint6
 
 // ---- gradients -----------------------------------------------------------------
 
-void Engine::load_margins(const float *m, uint64_t n, uint32_t outputs) {
-    if (n != n_rows_ * outputs) fail(kInvalid, "load_margins: length is not n_rows * n_outputs");
+// New margins of n values: nothing staged from the old ones holds.
+void Engine::reset_margins(uint64_t n, uint32_t outputs) {
     outputs_ = outputs;
     active_pairs_ = nullptr;
     row_pairs_live_ = false;
@@ -474,9 +474,57 @@ void Engine::load_margins(const float *m, uint64_t n, uint32_t outputs) {
     pair_array_stale_ = false;
     class_outputs_ = 0;
     margins_.resize(n);
-    margins_.upload(m, n, dev_.stream());
     if (poison_.size()) HBR_HIP(hipMemsetAsync(poison_.get(), 0, sizeof(uint32_t), dev_.stream()));
     labels_loaded_ = false;
+}
+
+void Engine::load_margins(const float *m, uint64_t n, uint32_t outputs) {
+    if (n != n_rows_ * outputs) fail(kInvalid, "load_margins: length is not n_rows * n_outputs");
+    reset_margins(n, outputs);
+    margins_.upload(m, n, dev_.stream());
+    dev_.sync();
+}
+
+void Engine::fill_margins(const std::vector<float> &base) {
+    const uint32_t k = (uint32_t)base.size();
+    const uint64_t n = n_rows_ * k;
+    reset_margins(n, k);
+    d_base_.reserve(k);
+    d_base_.upload(base.data(), k, dev_.stream());
+    FillArgs a{margins_.get(), d_base_.get(), n, k, 0u};
+    dev_.launch("hbr_fill_margins",
+                dim3(std::min<uint32_t>(ceil_div(n, kFoldThreads), (uint32_t)dev_.cu_count() * 2)), dim3(kFoldThreads), a);
+    dev_.sync();  // the upload has read `base`
+}
+
+std::vector<uint64_t> Engine::stage_labels(const float *labels, uint64_t n, uint32_t k) {
+    if (n != n_rows_) fail(kInvalid, "labels: one per row");
+    if (k > kSoftmaxMaxClasses) fail(kInvalid, "labels: too many values to count");
+    hipStream_t s = dev_.stream();
+    staged_labels_.resize(n);
+    staged_labels_.upload(labels, n, s);
+    static_assert(sizeof(unsigned long long) == sizeof(uint64_t), "label counts");
+    std::vector<uint64_t> counts(k, 0);
+    d_label_counts_.resize(k);
+    d_label_counts_.zero(s);
+    LabelArgs a{staged_labels_.get(), d_label_counts_.get(), n, k, 0u};
+    if (n)
+        dev_.launch("hbr_label_counts",
+                    dim3(std::min<uint32_t>(ceil_div(n, kFoldThreads), (uint32_t)dev_.cu_count())), dim3(kFoldThreads), a);
+    d_label_counts_.download(reinterpret_cast<unsigned long long *>(counts.data()), k, s);
+    dev_.sync();
+    return counts;
+}
+
+void Engine::take_labels(const float *weights, uint64_t n, bool binary) {
+    std::swap(labels_, staged_labels_);
+    has_weights_ = weights != nullptr;
+    if (weights) {
+        weights_.resize(n);
+        weights_.upload(weights, n, dev_.stream());
+    }
+    labels_binary_ = binary;
+    labels_loaded_ = true;
     dev_.sync();
 }
 
@@ -628,16 +676,13 @@ void Engine::order_rows_by_tree() {
     counters.row_orders++;
 }
 
+// The buffers stay with the engine for the next trainer's reorder (freeing
+// them took longer than the gathers).
 void Engine::restore_row_order() {
     if (!permuted_) return;
     gather_rows(perm_inv_.get());
     dev_.sync();
     permuted_ = false;
-    perm_.release();
-    perm_inv_.release();
-    group_stamp_.release();
-    bad_groups_.release();
-    spare_ = Spare{};
 }
 
 void Engine::read_gradients(float *out, uint64_t n) {

@@ -108,8 +108,16 @@ public:
     void prepare(const float *gpair, uint64_t n);
     // Device margins and labels (RowEngine::load_margins / gradients).
     void load_margins(const float *m, uint64_t n, uint32_t outputs);
+    void reset_margins(uint64_t n, uint32_t outputs);
     void set_labels(const float *labels, const float *weights, uint64_t n);
     bool labels_loaded() const { return labels_loaded_; }
+    // A trainer's start: its labels uploaded beside the engine's own and
+    // counted by value ([k]: labels equal to 0, 1, ..., k - 1); then every
+    // row's margins at `base` (one value an output) and the staged labels
+    // taken (binary: each is 0 or 1).
+    std::vector<uint64_t> stage_labels(const float *labels, uint64_t n, uint32_t k);
+    void fill_margins(const std::vector<float> &base);
+    void take_labels(const float *weights, uint64_t n, bool binary);
     // Gradients of output `output` from the device margins; false when some
     // gradient is not finite.
     bool compute_gradients(const hbr_device_loss &loss, uint32_t output);
@@ -534,6 +542,8 @@ private:
     DBuf<PartOut> g_pout_[2];
     QScale scale_host_{};
     bool grains_known_ = false;  // scale_host_.pad holds the staged pairs' grain codes
+    DBuf<float> staged_labels_, d_base_;  // stage_labels, fill_margins
+    DBuf<unsigned long long> d_label_counts_;
     DBuf<uint32_t> scalar_list_;  // rows the fused walk defers to hbr_finish_scale
     DBuf<uint32_t> rows_[2];
     DBuf<uint32_t> host_rows_;

@@ -1,5 +1,7 @@
 #include "trainer.h"
 
+#include "repeat_add.h"
+
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -395,9 +397,12 @@ Tree TreeBuilder::grow(std::vector<std::pair<Segment, float>> *leaves_out, bool 
 // the Hessian floor of the logistic and softmax losses (objective/mod.rs:150)
 constexpr float kMinHess = 1e-16f;
 
-static float weighted_label_mean(const float *labels, const float *weights, uint64_t n) {
+// counts: of the labels equal to 0 and to 1 (null: unknown).
+static float weighted_label_mean(const float *labels, const float *weights, uint64_t n, const uint64_t *counts) {
     double mean = 0.0;
-    if (weights) {
+    if (!weights && counts && n > 0 && counts[0] + counts[1] == n) {
+        mean = repeat_add(1.0 / (double)n, counts[1]);  // a label of 0 adds nothing
+    } else if (weights) {
         double sum_w = 0.0;
         for (uint64_t i = 0; i < n; i++) sum_w += (double)weights[i];
         if (sum_w > 0.0)
@@ -438,7 +443,8 @@ static float newton_step(bool logistic, const float *labels, const float *weight
     return (float)(-g / std::fmax(h, 1e-6));
 }
 
-std::vector<float> base_margins(const TrainParams &p, const float *labels, const float *weights, uint64_t n) {
+std::vector<float> base_margins(const TrainParams &p, const float *labels, const float *weights, uint64_t n,
+                                const uint64_t *counts) {
     if (p.objective == HBR_OBJ_SOFTMAX) {
         const uint32_t k = p.num_class;
         std::vector<float> m(k, 0.0f);
@@ -446,8 +452,12 @@ std::vector<float> base_margins(const TrainParams &p, const float *labels, const
             for (auto &v : m) v = p.base_score;
             return m;
         }
-        for (uint64_t i = 0; i < n; i++) {
-            if (labels[i] >= 0.0f && (uint32_t)labels[i] < k) m[(uint32_t)labels[i]] += weights ? weights[i] : 1.0f;
+        if (!weights && counts) {  // ones added in f32 stop at 2^24
+            for (uint32_t c = 0; c < k; c++) m[c] = (float)std::min<uint64_t>(counts[c], 1u << 24);
+        } else {
+            for (uint64_t i = 0; i < n; i++) {
+                if (labels[i] >= 0.0f && (uint32_t)labels[i] < k) m[(uint32_t)labels[i]] += weights ? weights[i] : 1.0f;
+            }
         }
         double sum_w = 0.0;
         if (weights)
@@ -472,14 +482,14 @@ std::vector<float> base_margins(const TrainParams &p, const float *labels, const
             if (raw) return {step};
             return {logit(1.0f / (std::exp(std::fmin(-step, 88.7f)) + 1.0f))};  // sigmoid_scalar, simd/mod.rs:425-427
         }
-        const float mean = weighted_label_mean(labels, weights, n);
+        const float mean = weighted_label_mean(labels, weights, n, counts);
         return {raw ? mean : logit(mean)};
     }
     // regression.rs:66-74: the Newton step when scale_pos_weight != 1
     if (p.has_base_score) return {p.base_score};
     if (std::fabs(p.scale_pos_weight - 1.0f) > 1e-6f)
         return {newton_step(false, labels, weights, n, p.scale_pos_weight)};
-    return {weighted_label_mean(labels, weights, n)};
+    return {weighted_label_mean(labels, weights, n, counts)};
 }
 
 Trainer::Trainer(Engine &e, const TrainParams &p, const float *labels, const float *weights, uint64_t n)
@@ -488,27 +498,22 @@ Trainer::Trainer(Engine &e, const TrainParams &p, const float *labels, const flo
     eval_owner_ = e.clear_eval_sets();  // an earlier trainer's sets would take this one's trees
     k_ = p.objective == HBR_OBJ_SOFTMAX ? p.num_class : 1;
     if (k_ == 0) fail(kInvalid, "softmax needs num_class");
-    if (p.objective == HBR_OBJ_SOFTMAX) {
-        if (k_ > kSoftmaxMaxClasses) fail(kRefused, "softmax: at most 1024 classes");
-        // multiclass.rs:96-100: class indices, non-negative integers below num_class
-        for (uint64_t i = 0; i < n; i++) {
-            const float y = labels[i];
-            if (!(y >= 0.0f && y < (float)k_) || y != std::floor(y))
-                fail(kInvalid, "softmax labels must be class indices below num_class");
-        }
-    }
-    labels_.assign(labels, labels + n);
-    if (weights) weights_.assign(weights, weights + n);
+    if (p.objective == HBR_OBJ_SOFTMAX && k_ > kSoftmaxMaxClasses) fail(kRefused, "softmax: at most 1024 classes");
+    // the labels go to the device once, which counts them per value (class);
+    // the engine's own labels change only below, when nothing is refused
+    const std::vector<uint64_t> counts = e_.stage_labels(labels, n, std::max(2u, k_));
+    uint64_t whole = 0;
+    for (uint32_t c = 0; c < (p.objective == HBR_OBJ_SOFTMAX ? k_ : 2u); c++) whole += counts[c];
+    // multiclass.rs:96-100: class indices, non-negative integers below num_class
+    if (p.objective == HBR_OBJ_SOFTMAX && whole != n)
+        fail(kInvalid, "softmax labels must be class indices below num_class");
     if (const char *v = std::getenv("HBROCM_SOFTMAX_BATCH")) softmax_batches = std::strtol(v, nullptr, 10) != 0;
-    base_ = base_margins(p, labels, weights, n);
+    base_ = base_margins(p, labels, weights, n, counts.data());
     // training/train.rs:425-433: a non-finite intercept is an error
     for (float b : base_)
         if (!std::isfinite(b)) fail(kInvalid, "estimated intercept is not finite; check the labels");
-    std::vector<float> m((size_t)n * k_);
-    for (uint64_t r = 0; r < n; r++)
-        for (uint32_t c = 0; c < k_; c++) m[r * k_ + c] = base_[c];
-    e_.load_margins(m.data(), m.size(), k_);
-    e_.set_labels(labels, weights, n);
+    e_.fill_margins(base_);
+    e_.take_labels(weights, n, counts[0] + counts[1] == n);
 }
 
 // Leaf values onto the margins (training/margins.rs:247-289): by routing

@@ -148,7 +148,6 @@ private:
     TrainParams p_;
     uint32_t k_ = 1;
     uint64_t n_;
-    std::vector<float> labels_, weights_;
     std::vector<float> base_;
     std::vector<Tree> trees_;
     uint64_t eval_owner_ = 0;  // the engine's eval-set owner number at construction
@@ -157,6 +156,8 @@ private:
 std::vector<GrowTreeNode> records_of(const Tree &t);
 
 // The loss's intercepts (objective base margins, train.rs:406-436).
-std::vector<float> base_margins(const TrainParams &p, const float *labels, const float *weights, uint64_t n);
+// counts: how many labels equal 0, 1, ..., num_class - 1 (at least two), or null.
+std::vector<float> base_margins(const TrainParams &p, const float *labels, const float *weights, uint64_t n,
+                                const uint64_t *counts = nullptr);
 
 }  // namespace hbr

@@ -84,3 +84,28 @@ def test_histogram_tiles_sum_every_row(n, f, bins, density):
     for c in (0, 1):
         want = np.bincount(row_bins, weights=pairs[rows, c].astype(np.float64), minlength=len(hist))
         assert np.array_equal(hist[:, c], want)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 1025, 300_001])
+def test_intercepts_from_counted_labels(n):
+    """The trainer's intercept from the device's label counts equals the
+    host's chain of additions over the labels, and labels that are not
+    classes are refused."""
+    rng = np.random.default_rng(n)
+    engine = hb.DMatrix(rng.standard_normal((n, 2), dtype=np.float32)).engine()
+    for y in ((rng.random(n) < 0.37).astype(np.float32), np.zeros(n, np.float32), np.full(n, -0.0, np.float32),
+              np.ones(n, np.float32), rng.standard_normal(n).astype(np.float32)):
+        mean = np.add.accumulate(y.astype(np.float64) / n)[-1]
+        for objective in ("reg:squarederror", "binary:logitraw"):
+            got = hb.Trainer(engine, {"objective": objective}, y).base_score()
+            assert got.view(np.uint32)[0] == np.float32(mean).view(np.uint32) or got[0] == np.float32(mean) == 0
+    k = 5
+    y = rng.integers(0, k, n).astype(np.float32)
+    t = hb.Trainer(engine, {"objective": "multi:softprob", "num_class": k}, y)
+    prior = np.log(np.float32(np.bincount(y.astype(int), minlength=k) / np.float32(n)) + np.float32(1e-6))
+    assert np.allclose(t.base_score(), prior - prior.mean(dtype=np.float32), rtol=0, atol=1e-5)
+    assert np.array_equal(t.margins().reshape(n, k), np.broadcast_to(t.base_score(), (n, k)))
+    for bad in (-1.0, float(k), 1.5, np.nan, np.inf):
+        y[n // 2] = bad
+        with pytest.raises(hb.HbrError):
+            hb.Trainer(engine, {"objective": "multi:softprob", "num_class": k}, y)
