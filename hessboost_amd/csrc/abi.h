@@ -343,7 +343,7 @@ struct HistNode {
     uint32_t contiguous; // rows are seg.offset .. seg.offset+len (no row buffer)
     uint32_t tile_begin; // first row tile (written by the plan kernel)
     uint32_t n_tiles;    // row tiles of the node (written by the plan kernel)
-    uint32_t pad[2];     // [0]: first partial of a multi-tile node; [1]: parent slot + 1 of a
+    uint32_t pad[2];     // [0]: first partial of a multi-tile node (of every node of a device-grown level); [1]: parent slot + 1 of a
                          // split's built child, whose sibling = parent - built as bins complete
                          // (dense kernels; both written by the plan kernel)
     uint32_t cls;        // class (tree) of a batched level: pairs at gpair + cls * class_rows,
@@ -366,7 +366,9 @@ struct PlanArgs {
     uint32_t *counts;           // [0] tiles, [1] tile_rows
     uint32_t min_cost;          // a tile's fixed cost in rows' (Engine::tile_cost)
     uint32_t fuse_subtract;     // built children of splits also update their siblings (dense kernels)
-    const GrowCounts *grow;     // non-null: one node per split of the level, n_splits read from here
+    // non-null: one node per split of the level, n_splits read from here; every
+    // node's tiles have partials
+    const GrowCounts *grow;
 };
 
 // The reference's CPU histogram in its own f64 order (replays): one
@@ -437,7 +439,7 @@ struct HistArgs {
     // fg) bins per (tile, feature group)
     const uint16_t *bins16;
     uint32_t stride16;          // elements per row (a multiple of 16)
-    uint32_t pad4;
+    uint32_t partials_only;     // every tile's sums to its partial, a one-tile node's too (hbr_reduce_scan)
 };
 
 // Dense indexes with a feature of more than 256 bins (at most kWideBinsMax):
@@ -496,7 +498,7 @@ struct ReduceArgs {
     uint32_t total_bins;
     uint32_t groups;
     uint32_t fg;
-    const GrowCounts *grow;     // non-null: nodes = its n_splits (the grid covers the most)
+    const GrowCounts *grow;     // hbr_reduce_scan: nodes = its n_splits (the grid covers the most)
     uint32_t group_bins;        // bins per feature in a partial: 256 (u8 rows) or kWideLdsBins / fg
     uint32_t quarters;          // workgroups per feature: group_bins / 64
 };
@@ -620,6 +622,12 @@ struct ScanArgs {
     uint32_t guard;          // 1: bound each candidate's error and flag near ties (kScanNearTie)
     uint32_t *cat_sets;
     uint32_t *best_sets;
+};
+
+// A level's reduce and search in one launch (hbr_reduce_scan).
+struct ReduceScanArgs {
+    ReduceArgs r;
+    ScanArgs s;
 };
 
 // ScanNode.pad flag: the node's total is on the device and its root gain is

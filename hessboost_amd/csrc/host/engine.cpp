@@ -1308,7 +1308,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     (void)host_nodes;
     d_htiles_.reserve(target + n);
     d_hcounts_.reserve(4);
-    d_partial_.reserve((size_t)(dense ? 2 * target : target + n) * groups * (dense ? fg * group_bins : kCsrGroupBins));
+    d_partial_.reserve((size_t)(dense ? 2 * target + (grow ? n : 0u) : target + n) * groups * (dense ? fg * group_bins : kCsrGroupBins));
 
     HistNode *nodes_rw = const_cast<HistNode *>(nodes_dev);  // the plan kernel resolves them in place
     PlanArgs p{};
@@ -1320,7 +1320,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     p.tiles = d_htiles_.get();
     p.counts = d_hcounts_.get();
     p.min_cost = tile_cost(groups);
-    p.fuse_subtract = dense ? 1u : 0u;
+    p.fuse_subtract = dense && !grow ? 1u : 0u;
     p.grow = grow;
     dev_.launch("hbr_hist_plan", dim3(1), dim3(256), p);
 
@@ -1352,6 +1352,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     a.min_hess = row_pairs_min_hess_;
     a.bins16 = rows16_.get();
     a.stride16 = stride16_;
+    a.partials_only = grow ? 1u : 0u;
     static const char *const wide_kernels[] = {"hbr_hist_dense16_fg1", "hbr_hist_dense16_fg2", "hbr_hist_dense16_fg4",
                                                "hbr_hist_dense16_fg8", "hbr_hist_dense16_fg16"};
     const char *k = wide ? wide_kernels[__builtin_ctz(fg)] : !dense_u8_ ? "hbr_hist_csr" : dense8_kernel(fg);
@@ -1366,7 +1367,8 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
         dev_.launch("hbr_hist_reduce_csr", dim3(ceil_div(total_bins_, 256), n), dim3(256), r);
     }
     if (dense) {
-        ReduceArgs r{};
+        ReduceArgs &r = reduce_args_;
+        r = ReduceArgs{};
         r.nodes = nodes_dev;
         r.partial = d_partial_.get();
         r.hist = hist_.get();
@@ -1378,7 +1380,8 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
         r.grow = grow;
         r.group_bins = group_bins;
         r.quarters = group_bins / 64u;
-        dev_.launch("hbr_hist_reduce", dim3(n_cols_ * r.quarters, n), dim3(1024), r);
+        // a device-grown level's partials are summed by its search
+        if (!grow) dev_.launch("hbr_hist_reduce", dim3(n_cols_ * r.quarters, n), dim3(1024), r);
     }
 }
 
@@ -1446,7 +1449,10 @@ void Engine::launch_scan(const ScanNode *nodes_dev, uint32_t n, const PartSplit 
         a.cat_sets = d_cat_sets_.get();
         a.best_sets = best_sets_dev;
     }
-    dev_.launch("hbr_scan_features", dim3(ceil_div(pairs, 4)), dim3(256), a);
+    if (grow)  // both children of each split; launch_hist left the reduce to it
+        dev_.launch("hbr_reduce_scan", dim3(n_cols_, n / 2), dim3(512), ReduceScanArgs{reduce_args_, a});
+    else
+        dev_.launch("hbr_scan_features", dim3(ceil_div(pairs, 4)), dim3(256), a);
     if (n_cat_) dev_.launch("hbr_scan_categorical", dim3(n * n_cat_), dim3(64), a);
     dev_.launch("hbr_scan_merge", dim3(n), dim3(256), a);
 }

@@ -376,6 +376,9 @@ private:
                      const GrowCounts *grow = nullptr);
     void launch_scan(const ScanNode *nodes_dev, uint32_t n, const PartSplit *splits_dev, const PartOut *part_out_dev,
                      ScanBest *best_dev, const GrowCounts *grow = nullptr, uint32_t *best_sets_dev = nullptr);
+    // the last launch_hist's reduce: a device-grown level's launch_scan does
+    // it in the same launch
+    ReduceArgs reduce_args_{};
     // the root's total, histogram and split search, queued (no synchronisation)
     void launch_root(const Segment &seg, uint32_t slot, float lower, float upper);
     // the roots of a device-grown batch (root t in slot t, of class t,

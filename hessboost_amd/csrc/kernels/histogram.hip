@@ -169,15 +169,17 @@ __device__ __forceinline__ void hist_dense8(const HistArgs &a) {
     }
     __syncthreads();
     const uint32_t *fo = a.feature_offset + f0;
-    QBin *dst = nd.n_tiles == 1 ? a.hist + (size_t)nd.slot * a.total_bins
-                                : a.partial + ((size_t)(nd.pad[0] + t.k) * a.groups + grp) * (FG * 256u);
+    // the level's search sums every tile's partial, a lone one's too
+    const bool whole = nd.n_tiles == 1 && !a.partials_only;
+    QBin *dst = whole ? a.hist + (size_t)nd.slot * a.total_bins
+                      : a.partial + ((size_t)(nd.pad[0] + t.k) * a.groups + grp) * (FG * 256u);
     for (uint32_t i = threadIdx.x; i < FG * 256u; i += blockDim.x) {
         // bin-major: consecutive threads read consecutive features (no bank conflicts)
         const uint32_t ff = BIN_MAJOR ? i % FG : i >> 8, bin = BIN_MAJOR ? i / FG : i & 255u;
         if (ff >= nf) continue;
         const uint32_t at = BIN_MAJOR ? i : ff * kLdsFeature + bin;
         const QBin v{(int64_t)lg[at], (int64_t)lh[at]};
-        if (nd.n_tiles == 1) {
+        if (whole) {
             const uint32_t lo = fo[ff], nb = fo[ff + 1] - lo;
             if (bin < nb) {
                 dst[lo + bin] = v;
@@ -359,7 +361,7 @@ extern "C" __global__ __launch_bounds__(256) void hbr_hist_plan(PlanArgs a) {
         const uint32_t n = (len + tile_rows - 1) / tile_rows;
         uint32_t all, part_all;
         const uint32_t first = block_exclusive_scan<256>(n, &all);
-        const uint32_t part_first = block_exclusive_scan<256>(n > 1 ? n : 0u, &part_all);
+        const uint32_t part_first = block_exclusive_scan<256>(n > 1 || a.grow ? n : 0u, &part_all);
         if (i < n_nodes) {
             a.nodes[i].tile_begin = carry + first;
             a.nodes[i].n_tiles = n;
@@ -510,7 +512,6 @@ extern "C" __global__ __launch_bounds__(1024) void hbr_hist_csr(HistArgs a) { hi
 extern "C" __global__ __launch_bounds__(1024) void hbr_hist_reduce(ReduceArgs a) {
     __shared__ int64_t acc[2][16][64];
     const uint32_t f = blockIdx.x / a.quarters, quarter = blockIdx.x % a.quarters;
-    if (a.grow && blockIdx.y >= a.grow->n_splits) return;
     const HistNode nd = a.nodes[blockIdx.y];
     if (f >= a.n_cols || nd.n_tiles == 1) return;  // uniform across the workgroup
     const uint32_t lo = a.feature_offset[f], nb = a.feature_offset[f + 1] - lo;

@@ -452,6 +452,186 @@ extern "C" __global__ __launch_bounds__(256) void hbr_scan_features(ScanArgs a) 
     }
 }
 
+// hbr_hist_reduce and hbr_scan_features of a level's splits in one launch,
+// for features of at most 256 bins: a workgroup per (split, feature) sums
+// the built child's partials (two slices of its tiles), takes the sibling
+// from the parent and stores both; then thread t searches bin t mod 256 of
+// child t / 256: its candidate of the forward pass and, where the bins miss
+// some of the node, of the backward pass (the suffix from a bin is the bins'
+// sum less the prefix before it). The candidates, their scores and the order
+// among equals are hbr_scan_features', which gives a lane four bins in turn.
+// Bound by its chain of dependent loads and f64 scores. A level of 100k x 32
+// rows takes 8.6 us where the two kernels took 4.6 + 8.4; of 10.5M x 28 rows
+// 13 us at 4 to 16 splits (8.3 + 9.5) and 26 at 64 (17.3 + 17.3).
+constexpr uint32_t kReduceScanThreads = 512;
+
+template <bool GUARD>
+__device__ __forceinline__ void reduce_scan(const ReduceScanArgs &ra) {
+    const ReduceArgs &r = ra.r;
+    const ScanArgs &a = ra.s;
+    constexpr uint32_t kWaves = kReduceScanThreads / kWave, kHalf = kWaves / 2;
+    __shared__ QBin s_bins[2][256];  // second slice's sums; then left child, right child
+    __shared__ QBin s_sum[kWaves];
+    __shared__ float s_loss[kWaves], s_rival[kWaves];
+    __shared__ uint32_t s_idx[kWaves], s_nan[kWaves];
+    __shared__ QBin s_win[2];
+    const uint32_t f = blockIdx.x, split = blockIdx.y;
+    const uint32_t child = threadIdx.x >> 8, bin = threadIdx.x & 255u;
+    const uint32_t lane = lane_id(), wave = threadIdx.x / kWave, wave0 = child * kHalf;
+    // every record the workgroup may need, loaded at once (the arrays hold
+    // the most splits the level can have)
+    const uint32_t lo = r.feature_offset[f], nb = r.feature_offset[f + 1] - lo;
+    const HistNode hn = r.nodes[split];
+    const PartSplit sp = a.splits[split];
+    const PartOut po = a.part_out[split];
+    const ScanNode nd = a.nodes[2 * split + child];
+    if (split >= r.grow->n_splits) return;  // uniform across the workgroup
+    const uint32_t cls = nd.pad >> kScanClassShift;
+    const int eg = a.scale[cls].exp_g, eh = a.scale[cls].exp_h;
+    QBin *built = r.hist + (size_t)hn.slot * r.total_bins + lo;
+    QBin *par = r.hist + (size_t)sp.parent_slot * r.total_bins + lo;
+    const bool in = bin < nb;
+    QBin q{0, 0}, pv{0, 0};
+    if (child == 0 && in) pv = par[bin];
+    if (in) {
+        const uint32_t grp = f / r.fg, local = (f % r.fg) * r.group_bins + bin;
+        const size_t step = (size_t)r.groups * (r.fg * r.group_bins);
+        const QBin *src = r.partial + (size_t)hn.pad[0] * step + (size_t)grp * (r.fg * r.group_bins) + local;
+#pragma unroll 4
+        for (uint32_t k = child; k < hn.n_tiles; k += 2) {
+            const QBin v = src[k * step];
+            q.g += v.g;
+            q.h += v.h;
+        }
+    }
+    if (child == 1) s_bins[0][bin] = q;
+    __syncthreads();
+    const uint32_t built_right = po.left_len <= po.right_len ? 0u : 1u;
+    if (child == 0) {
+        q.g += s_bins[0][bin].g;
+        q.h += s_bins[0][bin].h;
+        pv.g -= q.g;
+        pv.h -= q.h;
+        if (in) {
+            built[bin] = q;
+            par[bin] = pv;
+        }
+        s_bins[built_right][bin] = q;  // this thread alone read s_bins[0][bin]
+        s_bins[1u - built_right][bin] = pv;
+    }
+    __syncthreads();
+    const QBin mine = s_bins[child][bin];
+    const int64_t ig = wave_inclusive_scan(mine.g), ih = wave_inclusive_scan(mine.h);
+    if (lane == kWave - 1) s_sum[wave] = QBin{ig, ih};
+    __syncthreads();
+    int64_t ag = ig, ah = ih, fg = 0, fh = 0;  // the prefix, and the bins' sum
+#pragma unroll
+    for (uint32_t w = 0; w < kHalf; w++) {
+        const QBin t = s_sum[wave0 + w];
+        if (wave0 + w < wave) {
+            ag += t.g;
+            ah += t.h;
+        }
+        fg += t.g;
+        fh += t.h;
+    }
+    const int64_t tg = nd.total.g, th = nd.total.h;
+    const int dir = a.monotone ? (int)a.monotone[f] : 0;
+    Bound bound{0.0, 0.0};
+    if (GUARD)
+        bound = node_bound(child == 0 ? po.left_len : po.right_len, eg, eh, __uint_as_float(a.scale[cls].max_g_bits),
+                           __uint_as_float(a.scale[cls].max_h_bits));
+    Cand best;
+    best.loss = -__builtin_inff();
+    best.idx = 0xffffffffu;
+    best.lg = best.lh = best.rg = best.rh = 0;
+    best.backward = 0;
+    best.err = 0.0f;
+    best.fragile = 0;
+    bool nan_seen = false;
+    Rivals riv;
+    riv.init();
+    auto consider = [&](int64_t lg, int64_t lh, uint32_t idx, uint32_t backward) {
+        float loss;
+        if (GUARD) {
+            const Scored sc = score_guarded(dequant(lg, eg), dequant(lh, eh), dequant(tg - lg, eg), dequant(th - lh, eh),
+                                            a.reg, nd.lower, nd.upper, dir, nd.root_gain, bound);
+            if (sc.ok) offer(best, nan_seen, sc.loss, idx, lg, lh, tg - lg, th - lh, backward, sc.err, sc.fragile);
+            if (sc.rival) riv.offer(up32((double)sc.loss + (double)sc.err), lg, lh);
+        } else if (score(dequant(lg, eg), dequant(lh, eh), dequant(tg - lg, eg), dequant(th - lh, eh), a.reg, nd.lower,
+                         nd.upper, dir, nd.root_gain, &loss)) {
+            offer(best, nan_seen, loss, idx, lg, lh, tg - lg, th - lh, backward);
+        }
+    };
+    if (in && nb > 1) {
+        consider(ag, ah, bin, 0u);
+        if (!a.dense && (fg != tg || fh != th))  // the suffix from this bin on the right
+            consider(tg - (fg - (ag - mine.g)), th - (fh - (ah - mine.h)), nb + (nb - 1 - bin), 1u);
+    }
+    // the child's best: highest loss, then lowest candidate index
+    float bl = best.loss;
+    uint32_t bi = best.idx;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        const float ol = __shfl_xor(bl, d, kWave);
+        const uint32_t oi = (uint32_t)__shfl_xor((int)bi, d, kWave);
+        if (better(ol, oi, bl, bi)) {
+            bl = ol;
+            bi = oi;
+        }
+    }
+    const uint64_t any_nan = __ballot(nan_seen);
+    if (lane == 0) {
+        s_loss[wave] = bl;
+        s_idx[wave] = bi;
+        s_nan[wave] = any_nan ? kScanNumericNaN : 0u;
+    }
+    __syncthreads();
+    uint32_t nan_flag = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kHalf; w++) {
+        const float ol = s_loss[wave0 + w];
+        const uint32_t oi = s_idx[wave0 + w];
+        if (better(ol, oi, bl, bi)) {
+            bl = ol;
+            bi = oi;
+        }
+        nan_flag |= s_nan[wave0 + w];
+    }
+    const bool won = bi != 0xffffffffu, winner = won && best.idx == bi;
+    float rival = -__builtin_inff();
+    if (GUARD) {
+        if (winner) s_win[child] = QBin{best.lg, best.lh};
+        __syncthreads();
+        const QBin w = s_win[child];
+        rival = won ? riv.excluding(w.g, w.h) : riv.top;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) rival = fmaxf(rival, __shfl_xor(rival, d, kWave));
+        if (lane == 0) s_rival[wave] = rival;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t w2 = 0; w2 < kHalf; w2++) rival = fmaxf(rival, s_rival[wave0 + w2]);
+    }
+    if (winner || (!won && bin == 0)) {
+        ScanBest o;
+        o.loss = won ? bl : -__builtin_inff();
+        o.feature = f;
+        o.index = bi;
+        o.flags = nan_flag;
+        o.left = QBin{best.lg, best.lh};
+        o.right = QBin{best.rg, best.rh};
+        o.err = best.err;
+        o.rival = rival;
+        if (won) o.flags |= best.backward | (best.fragile ? kScanNearTie : 0u);
+        a.per_feature[(size_t)(2 * split + child) * a.n_features + f] = o;
+    }
+}
+
+extern "C" __global__ __launch_bounds__(kReduceScanThreads, 4) void hbr_reduce_scan(ReduceScanArgs ra) {
+    if (ra.s.guard) reduce_scan<true>(ra);
+    else reduce_scan<false>(ra);
+}
+
 // The feature-order merge of a node's per-feature winners (`per_node`,
 // n_features records), by one workgroup of kMergeThreads: thread t takes
 // features t, t + kMergeThreads, ... (ascending, so within a thread only a

@@ -109,3 +109,20 @@ def test_intercepts_from_counted_labels(n):
         y[n // 2] = bad
         with pytest.raises(hb.HbrError):
             hb.Trainer(engine, {"objective": "multi:softprob", "num_class": k}, y)
+
+
+# one to several groups of features and tiles, narrow and constant features,
+# missing cells (the backward pass), with and without the guard, monotone
+@pytest.mark.parametrize("n,f,nan,params", [
+    (300, 1, 0.0, {}), (5_000, 3, 0.2, {}), (40_000, 33, 0.0, {"gamma": 0.1, "monotone_constraints": [1, -1]}),
+    (40_000, 33, 0.1, {"monotone_constraints": [1, -1], "min_child_weight": 3.0}), (120_000, 70, 0.05, {"alpha": 0.2}),
+    (9_000, 4, 0.3, {"max_bin": 17}), (9_000, 5, 0.0, {"max_delta_step": 0.4}),
+])
+def test_level_reduce_and_search_give_the_host_levels_trees(monkeypatch, n, f, nan, params):
+    x, y = _data(n, f, nan, seed=n + f)
+    x[:, -1] = 3.0  # one bin: no candidate
+    x[:, f // 2] = np.round(x[:, f // 2])
+    params = dict(params, objective="binary:logistic", max_depth=7, eta=0.3)
+    device, host = _both(monkeypatch, x, y, params, 2)
+    assert device[2].get("hbr_reduce_scan", 0) > 0
+    _same(device, host)
