@@ -1308,7 +1308,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     (void)host_nodes;
     d_htiles_.reserve(target + n);
     d_hcounts_.reserve(4);
-    d_partial_.reserve((size_t)(dense ? 2 * target + (grow ? n : 0u) : target + n) * groups * (dense ? fg * group_bins : kCsrGroupBins));
+    d_partial_.reserve((size_t)(2 * target + (grow ? n : 0u)) * groups * (dense ? fg * group_bins : kCsrGroupBins));
 
     HistNode *nodes_rw = const_cast<HistNode *>(nodes_dev);  // the plan kernel resolves them in place
     PlanArgs p{};

@@ -306,6 +306,7 @@ public:
     uint32_t alloc_slot();
     void free_slot(uint32_t s);
     bool reserve_slots(uint64_t n);
+    size_t free_slots() const { return free_slots_.size(); }
 
     // scan regularization and monotone directions for the next scans
     void set_scan_params(const ScanParams &p, const std::vector<int8_t> &monotone);

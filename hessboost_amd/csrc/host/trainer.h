@@ -13,6 +13,7 @@
 // gradients of the device margins, one tree per output, and each leaf's
 // value added to its rows' margins.
 #pragma once
+#include <deque>
 #include <cstdint>
 #include <vector>
 
@@ -77,6 +78,10 @@ private:
         ScanBest best;
         std::array<uint32_t, kCatWords> best_set;  // a categorical winner's local bins
         bool searched;
+        int32_t ahead = -1;  // best-first: its children, once split (index of ahead_)
+    };
+    struct Ahead {
+        Open kids[2];
     };
     struct Decision {
         bool valid = false;
@@ -92,6 +97,12 @@ private:
         const std::array<uint32_t, kCatWords> *set = nullptr;
     };
     Decision decide(const Open &o) const;
+    void child_bounds_of(const Open &o, const Decision &d, double cb[4]) const;
+    void leaf_rows(int32_t nid, const Open &o);
+    LevelSplit split_of(const Open &o, const Decision &d, double cb[4]) const;
+    std::vector<uint32_t> set_codes(const Decision &d) const;
+    void record(Tree &t, const Open &o, const Decision &d, const double cb[4]);
+    void split_ahead(Open &o, std::vector<Open> &heap, uint64_t leaves_left, uint64_t limit);
     // Expand node o by d: children appended to the tree; returns the level split.
     LevelSplit expand(Tree &t, const Open &o, const Decision &d, double cb[4]);
     void leaf(const Open &o);
@@ -103,6 +114,8 @@ private:
     // per node id
     std::vector<double> g_, h_, lower_, upper_;
     std::vector<std::pair<int32_t, Segment>> leaves_;
+    std::deque<Ahead> ahead_;
+    bool speculate_ = false;
 };
 
 struct TrainParams {

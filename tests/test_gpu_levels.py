@@ -126,3 +126,31 @@ def test_level_reduce_and_search_give_the_host_levels_trees(monkeypatch, n, f, n
     device, host = _both(monkeypatch, x, y, params, 2)
     assert device[2].get("hbr_reduce_scan", 0) > 0
     _same(device, host)
+
+
+# best-first trees whose nodes are split ahead of their pops: budgets that end
+# before, inside and after a batch, more leaves than the rows allow; dense
+# rows (margins by the walk) and sparse ones (margins by each leaf's rows)
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("leaves,depth", [(2, 0), (3, 0), (6, 0), (40, 0), (41, 5), (200, 0), (0, 4), (5000, 0)])
+def test_best_first_trees_split_ahead_match_the_oracle(sparse, leaves, depth):
+    from oracle import oracle as O
+    from tests.test_gpu_train import compare_trees
+
+    rng = np.random.default_rng(leaves + 7 * depth)
+    n, f = 3_000, 30
+    x = rng.exponential(1.0, (n, f)).astype(np.float32)
+    if sparse:
+        x[rng.random(x.shape) < 0.85] = np.nan
+    y = (np.nan_to_num(x[:, 0]) - np.nan_to_num(x[:, 1]) * np.nan_to_num(x[:, 2]) + rng.standard_normal(n) * 0.1)
+    y = y.astype(np.float32)
+    params = {"grow_policy": "lossguide", "max_depth": depth, "max_leaves": leaves, "eta": 0.3, "min_child_weight": 2.0}
+    ref = O.Model(O.Dataset(x), y, O.params(grow_policy=O.GROW_LOSSGUIDE, max_depth=depth, max_leaves=leaves,
+                                            min_child_weight=2.0), 3)
+    engine = hb.DMatrix(x, label=y).engine()
+    t = hb.Trainer(engine, params, y)
+    before = engine.counters()
+    t.boost(3)
+    compare_trees(t.trees(), ref.trees())
+    assert np.max(np.abs(t.margins() - ref.margins().reshape(-1))) <= 1e-5
+    assert engine.counters()["near_ties"] - before["near_ties"] <= sum(len(k["left"]) for k in t.trees())
