@@ -316,7 +316,8 @@ struct PartArgs {
     const GrowCounts *grow;      // non-null: n_splits and n_tiles are read from here
     const uint32_t *tile_split;  // non-null: the split of every tile (else found by binary search)
     uint32_t csr_ascending;      // every CSR row's global bins ascend: routing binary-searches them
-    uint32_t pad;
+    uint32_t csr_groups;         // bin ranges of csr_ranges
+    const uint32_t *csr_ranges;  // each row's first entry of every bin range (HistArgs::csr_ranges) or null
     const uint32_t *cat_tables;  // kCatWords words per categorical split: its left local bins
     uint32_t move_tile;          // hbr_part_move: rows per tile (kMoveRows x its threads)
     uint32_t pad2;
@@ -423,7 +424,7 @@ struct HistArgs {
     uint32_t total_bins;
     uint32_t groups;            // feature groups (dense) or bin ranges (CSR) per tile
     uint32_t class_rows;        // batched levels: the pairs of class c start at gpair + c * class_rows
-    uint32_t pad;
+    uint32_t csr_lanes;         // CSR: lanes a row (a power of two, 4 to 64)
     // CSR rows whose global bins ascend: row r's entries of bin range g are
     // row_ptr[r] + [csr_ranges[r * (groups + 1) + g], ... + g + 1]) (null: scan the row)
     const uint32_t *csr_ranges;

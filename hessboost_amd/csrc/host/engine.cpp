@@ -1283,6 +1283,15 @@ uint32_t Engine::tile_cost(uint32_t groups) const {
     return groups * (dense16_ ? 22u : dense_u8_ ? 11u : 2u);
 }
 
+// Lanes a row of the CSR histogram: the entries a workgroup reads of an
+// average row (its range's, or all), rounded up to a power of two.
+uint32_t Engine::csr_lanes(uint32_t groups, bool ranges) const {
+    const uint64_t per_row = n_rows_ ? entries_ / n_rows_ / (ranges ? groups : 1) + 1 : 1;
+    uint32_t lanes = 4;
+    while (lanes < 64 && lanes < per_row) lanes *= 2;
+    return lanes;
+}
+
 // Histograms of a batch of nodes into their slots: the plan kernel cuts the
 // nodes' rows into tiles (about `per_cu` resident workgroups per CU over the
 // launch), then one workgroup per (tile, feature group). Dense u8 tiles
@@ -1334,6 +1343,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     a.scale = level_scale_ ? level_scale_ : scale_dev();
     a.class_rows = level_pairs_ ? (uint32_t)n_rows_ : 0u;
     a.csr_ranges = !dense_u8_ && csr_ranges_.size() ? csr_ranges_.get() : nullptr;
+    a.csr_lanes = csr_lanes(groups, a.csr_ranges != nullptr);
     a.bins8 = rows8_.get();
     a.stride = stride_;
     a.n_cols = n_cols_;
@@ -1530,6 +1540,8 @@ PartArgs Engine::part_args() const {
     a.row_ptr = row_ptr_.get();
     a.gbins = gbins_.get();
     a.csr_ascending = csr_ascending_ ? 1u : 0u;
+    a.csr_ranges = csr_ranges_.size() ? csr_ranges_.get() : nullptr;
+    a.csr_groups = ceil_div(total_bins_, kCsrGroupBins);
     a.feature_offset = d_fo_.get();
     a.n_rows = (uint32_t)n_rows_;
     a.words = words_;
@@ -2486,6 +2498,7 @@ bool Engine::build_rows_fixed(const uint32_t *rows, uint64_t m, double *out, uin
     a.scale = f.scale;
     a.class_rows = level_pairs_ ? (uint32_t)n_rows_ : 0u;
     a.csr_ranges = !dense_u8_ && csr_ranges_.size() ? csr_ranges_.get() : nullptr;
+    a.csr_lanes = csr_lanes(groups, a.csr_ranges != nullptr);
     a.bins8 = rows8_.get();
     a.stride = stride_;
     a.n_cols = n_cols_;

@@ -423,6 +423,7 @@ private:
     PartArgs part_args() const;
     uint32_t part_move_threads(uint64_t rows) const;
     uint32_t tile_cost(uint32_t groups) const;
+    uint32_t csr_lanes(uint32_t groups, bool ranges) const;
     void scan_host_nodes(const std::vector<ScanNode> &nodes, ScanBest *out, uint32_t *sets = nullptr);
     void launch_gradients(const hbr_device_loss &loss, uint32_t output);
     GradArgs grad_args(const hbr_device_loss &loss);

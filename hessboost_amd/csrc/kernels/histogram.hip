@@ -196,13 +196,16 @@ __device__ __forceinline__ void hist_dense8(const HistArgs &a) {
 }
 
 // Sparse rows into one range of kCsrGroupBins global bins, privately in
-// LDS: the workgroup's 16 waves take the tile's rows, each wave four rows
-// at a time (their row pointers, pairs and entries loaded together), its
-// lanes 64 entries of a row at a time; an entry in the range adds its
-// row's quantised pair with LDS atomics. Then the range goes to the node's
-// slot (a node of one tile) or to the tile's partial, summed by
-// hbr_hist_reduce_csr. Every range of every tile is written, so slots need
-// no zeroing.
+// LDS: the workgroup's 16 waves take the tile's rows, a.csr_lanes lanes a
+// row and kCsrRows rows a lane at a time (their row pointers, pairs and
+// entries loaded together); an entry in the range adds its row's quantised
+// pair with LDS atomics. A row holds few entries of a range (100 entries
+// over 31 ranges: 3), so a wave of one row at a time left 60 lanes idle
+// and waited for its chain of loads (id, pointer, range, entries) alone: the
+// root of 100k x 1,000 sparse rows took 1,119 us, with 4 lanes a row 119.
+// Then the range goes to the node's slot (a node of one tile) or to the
+// tile's partial, summed by hbr_hist_reduce_csr. Every range of every tile
+// is written, so slots need no zeroing.
 constexpr uint32_t kCsrRows = 4;
 
 __device__ __forceinline__ void hist_csr(const HistArgs &a) {
@@ -219,33 +222,38 @@ __device__ __forceinline__ void hist_csr(const HistArgs &a) {
     const GPair *gpair = a.gpair + (size_t)nd.cls * a.class_rows;
     const uint32_t *rows = a.rows[nd.seg.buf] + nd.seg.offset;
     const uint32_t end = t.row0 + t.rows;
-    const uint32_t wave = threadIdx.x / kWave, waves = blockDim.x / kWave, lane = lane_id();
-    for (uint32_t j0 = t.row0 + wave; j0 < end; j0 += kCsrRows * waves) {
+    const uint32_t step = blockDim.x / a.csr_lanes;  // rows the workgroup takes at once
+    const uint32_t sub = threadIdx.x % a.csr_lanes;
+    // whole waves stay in the loop (the entry loop's length is the wave's)
+    for (uint32_t base = t.row0; base < end; base += kCsrRows * step) {
         uint64_t b[kCsrRows], e[kCsrRows];
         unsigned long long qg[kCsrRows], qh[kCsrRows];
         uint32_t iters = 0;
 #pragma unroll
         for (uint32_t u = 0; u < kCsrRows; u++) {
-            const uint32_t j = j0 + u * waves;
+            const uint32_t j = base + u * step + threadIdx.x / a.csr_lanes;
             const bool ok = j < end;
             const uint32_t r = ok ? (nd.contiguous ? nd.seg.offset + j : rows[j]) : 0u;
             b[u] = ok ? a.row_ptr[r] : 0ull;
-            e[u] = ok ? a.row_ptr[r + 1] : 0ull;
-            if (ok && a.csr_ranges) {  // only this range's entries
+            if (a.csr_ranges) {  // only this range's entries
                 const uint32_t *rg = a.csr_ranges + (size_t)r * (a.groups + 1) + grp;
-                e[u] = b[u] + rg[1];
-                b[u] += rg[0];
+                e[u] = ok ? b[u] + rg[1] : 0ull;
+                b[u] += ok ? rg[0] : 0u;
+            } else {
+                e[u] = ok ? a.row_ptr[r + 1] : 0ull;
             }
             const GPair p = ok ? gpair[r] : GPair{0.0f, 0.0f};
             qg[u] = (unsigned long long)quantize(p.g, eg);
             qh[u] = (unsigned long long)quantize(p.h, eh);
-            iters = max(iters, (uint32_t)((e[u] - b[u] + kWave - 1) / kWave));
+            iters = max(iters, (uint32_t)((e[u] - b[u] + a.csr_lanes - 1) / a.csr_lanes));
         }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) iters = max(iters, (uint32_t)__shfl_xor((int)iters, d, kWave));
         for (uint32_t k = 0; k < iters; k++) {
             uint32_t d[kCsrRows];
 #pragma unroll
             for (uint32_t u = 0; u < kCsrRows; u++) {
-                const uint64_t x = b[u] + (uint64_t)k * kWave + lane;
+                const uint64_t x = b[u] + (uint64_t)k * a.csr_lanes + sub;
                 d[u] = x < e[u] ? a.gbins[x] - lo_bin : 0xffffffffu;
             }
 #pragma unroll

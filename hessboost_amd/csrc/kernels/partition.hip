@@ -38,26 +38,11 @@ __device__ __forceinline__ bool goes_left(const PartArgs &a, const PartSplit &sp
         const uint32_t local = a.cols8 ? (uint32_t)a.cols8[at] : (uint32_t)a.cols16[at];
         return present_left(a, sp, local);
     }
-    // a row's global bins ascend (its entries are in feature order, and a
-    // feature's bins follow the previous feature's): the first bin >= fs,
-    // by binary search, is the feature's entry if it lies below fe
+    // sparse rows in the caller's order (ascending ones: route_csr)
     const uint32_t fs = a.feature_offset[sp.feature], fe = a.feature_offset[sp.feature + 1];
-    if (!a.csr_ascending) {  // entries in the caller's order: scan them
-        for (uint64_t e = a.row_ptr[r]; e < a.row_ptr[r + 1]; e++) {
-            const uint32_t gb = a.gbins[e];
-            if (gb >= fs && gb < fe) return present_left(a, sp, gb - fs);
-        }
-        return sp.default_left != 0;
-    }
-    uint64_t lo = a.row_ptr[r], hi = a.row_ptr[r + 1];
-    while (lo < hi) {
-        const uint64_t mid = lo + (hi - lo) / 2;
-        if (a.gbins[mid] < fs) lo = mid + 1;
-        else hi = mid;
-    }
-    if (lo < a.row_ptr[r + 1]) {
-        const uint32_t gb = a.gbins[lo];
-        if (gb < fe) return present_left(a, sp, gb - fs);
+    for (uint64_t e = a.row_ptr[r]; e < a.row_ptr[r + 1]; e++) {
+        const uint32_t gb = a.gbins[e];
+        if (gb >= fs && gb < fe) return present_left(a, sp, gb - fs);
     }
     return sp.default_left != 0;
 }
@@ -111,6 +96,56 @@ __device__ __forceinline__ void route_dense8(const PartArgs &a, const PartSplit 
     }
 }
 
+// The same for sparse rows whose global bins ascend: the eight rows' searches
+// step together (eight loads in flight a step), among the entries of the
+// feature's bin ranges where the index keeps their starts.
+__device__ __forceinline__ void route_csr(const PartArgs &a, const PartSplit &sp, const uint32_t (&r)[kRowsPerThread],
+                                          bool (&left)[kRowsPerThread]) {
+    const uint32_t fs = a.feature_offset[sp.feature], fe = a.feature_offset[sp.feature + 1];
+    const uint32_t g0 = fs / kCsrGroupBins, g1 = (fe - 1) / kCsrGroupBins + 1;
+    uint64_t lo[kRowsPerThread], hi[kRowsPerThread], end[kRowsPerThread];
+#pragma unroll
+    for (uint32_t k = 0; k < kRowsPerThread; k++) {
+        lo[k] = end[k] = 0;
+        if (r[k] == 0xffffffffu || fs == fe) continue;
+        const uint64_t b = a.row_ptr[r[k]];
+        if (a.csr_ranges) {
+            const uint32_t *rg = a.csr_ranges + (size_t)r[k] * (a.csr_groups + 1);
+            lo[k] = b + rg[g0];
+            end[k] = b + rg[g1];
+        } else {
+            lo[k] = b;
+            end[k] = a.row_ptr[r[k] + 1];
+        }
+    }
+    bool more = false;
+#pragma unroll
+    for (uint32_t k = 0; k < kRowsPerThread; k++) {
+        hi[k] = end[k];
+        more |= lo[k] < hi[k];
+    }
+    while (more) {
+        uint32_t gb[kRowsPerThread];
+#pragma unroll
+        for (uint32_t k = 0; k < kRowsPerThread; k++) gb[k] = lo[k] < hi[k] ? a.gbins[lo[k] + (hi[k] - lo[k]) / 2] : 0u;
+        more = false;
+#pragma unroll
+        for (uint32_t k = 0; k < kRowsPerThread; k++) {
+            if (lo[k] >= hi[k]) continue;
+            const uint64_t mid = lo[k] + (hi[k] - lo[k]) / 2;
+            if (gb[k] < fs) lo[k] = mid + 1;
+            else hi[k] = mid;
+            more |= lo[k] < hi[k];
+        }
+    }
+    uint32_t gb[kRowsPerThread];
+#pragma unroll
+    for (uint32_t k = 0; k < kRowsPerThread; k++) gb[k] = lo[k] < end[k] ? a.gbins[lo[k]] : 0xffffffffu;
+#pragma unroll
+    for (uint32_t k = 0; k < kRowsPerThread; k++)
+        left[k] = r[k] != 0xffffffffu && (gb[k] < fe ? present_left(a, sp, gb[k] - fs) : sp.default_left != 0);
+}
+
 // Count pass: each wave's 64-row ballots of "goes left" and the tile's left
 // count. The row ids, then the routing bytes, are loaded eight at a time.
 extern "C" __global__ __launch_bounds__(256) void hbr_part_count(PartArgs a) {
@@ -135,6 +170,8 @@ extern "C" __global__ __launch_bounds__(256) void hbr_part_count(PartArgs a) {
     if (a.dense && a.cols8) {
         if (a.missing) route_dense8<true>(a, sp, r, left);
         else route_dense8<false>(a, sp, r, left);
+    } else if (!a.dense && a.csr_ascending) {
+        route_csr(a, sp, r, left);
     } else {
 #pragma unroll
         for (uint32_t k = 0; k < kRowsPerThread; k++) left[k] = r[k] != 0xffffffffu && goes_left(a, sp, r[k]);
