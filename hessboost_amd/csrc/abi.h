@@ -956,6 +956,10 @@ struct alignas(8) CompactNode {
 // reads row l of every feature from bank l, whatever the feature.
 constexpr uint32_t kPredPitch = 64;
 
+// LDS a wave of the shared pair walk leaves its 16 trees' values of a 64-row
+// block in.
+constexpr uint32_t kPairTreeBytes = 16 * kPredPitch * 4;
+
 // Two levels of a complete tree (PredictArgs::pairs).
 struct alignas(16) PairRecord {
     uint32_t t_node, t_first, t_second;
@@ -1036,8 +1040,14 @@ struct PredictArgs {
     // is continued by nodes that read slot 0 (NaN) and so always take their
     // first child, down to its position at level D, which holds its value.
     const PairRecord *pairs;
+    // The trees stand in the order of their outputs (a tree's margin only
+    // meets those of its output, whose order is kept).
     const uint32_t *pair_values;   // n_trees x 2^D leaf values (bits)
     const int32_t *pair_orig;      // n_trees x 2^D: the caller's id of the leaf each position holds
+    const uint32_t *pair_tree;     // n_trees: the caller's number of each tree
+    const uint32_t *pair_output;   // n_trees, ascending
+    const uint32_t *pair_first;    // n_outputs + 1: each output's first tree
+    const float *pair_weight;      // n_trees
 };
 constexpr uint32_t kPredCategorical = 1u << 29;
 

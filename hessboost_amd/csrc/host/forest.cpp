@@ -172,8 +172,15 @@ void Forest::build_pairs(const hbr_forest_desc &fd) {
     std::vector<uint32_t> values(n_trees_ * leaves);
     std::vector<int32_t> orig(n_trees_ * leaves);
     std::vector<uint32_t> t_at, s_at;  // per complete position of levels < depth
+    std::vector<uint32_t> order(n_trees_), outputs(n_trees_);
+    std::vector<float> weights(n_trees_);
+    auto output_of = [&](uint32_t t) { return fd.tree_output ? fd.tree_output[t] : 0u; };
+    for (uint32_t t = 0; t < n_trees_; t++) order[t] = t;
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return output_of(x) < output_of(y); });
     for (uint64_t t = 0; t < n_trees_; t++) {
-        const uint64_t lo = fd.tree_offset[t];
+        outputs[t] = output_of(order[t]);
+        weights[t] = fd.tree_weight ? fd.tree_weight[order[t]] : 1.0f;
+        const uint64_t lo = fd.tree_offset[order[t]];
         t_at.assign((1ull << depth) - 1, 0u);
         s_at.assign((1ull << depth) - 1, 0u);  // slot 0, m 0: the first child
         // (node, level, position in its level)
@@ -224,6 +231,18 @@ void Forest::build_pairs(const hbr_forest_desc &fd) {
     pair_values_.upload(values.data(), values.size(), s);
     pair_orig_.resize(orig.size());
     pair_orig_.upload(orig.data(), orig.size(), s);
+    pair_tree_.resize(n_trees_);
+    pair_tree_.upload(order.data(), n_trees_, s);
+    pair_output_.resize(n_trees_);
+    pair_output_.upload(outputs.data(), n_trees_, s);
+    std::vector<uint32_t> first(n_outputs_ + 1);
+    for (uint32_t o = 0; o <= n_outputs_; o++)
+        first[o] = (uint32_t)(std::lower_bound(outputs.begin(), outputs.end(), o) - outputs.begin());
+    pair_first_.resize(first.size());
+    pair_first_.upload(first.data(), first.size(), s);
+    pair_weight_.resize(n_trees_);
+    pair_weight_.upload(weights.data(), n_trees_, s);
+    dev_.sync();  // the uploads have read this call's arrays
     pair_levels_ = levels;
     pairs_ok_ = true;
 }
@@ -281,6 +300,50 @@ void Forest::build_mirror(const hbr_forest_desc &fd) {
     mirror_ok_ = true;
 }
 
+// Waves a workgroup of the pair walk shares its 64-row block among (1: a wave
+// a block, its trees' sums in registers). A wave keeps 16 trees in flight and
+// the kernels' registers allow 16 waves a CU, so sharing pays where fewer
+// would run:
+// - up to four blocks a CU: enough waves for 16 (one block of 28 features and
+//   100 trees 47 -> 24 us; 1,024 blocks 54 -> 39; 100 features, 1,000 trees
+//   346 -> 73 and 411 -> 268; 2,048 blocks of 28 features 57 -> 60);
+// - else, for 256 trees or more, row blocks of which LDS holds fewer than 16:
+//   the fewest waves that bring more than 12 to a CU (2^20 rows, 1,000 trees:
+//   50 features 3,977 -> 3,201 us, 70 features 5,315 -> 3,299, 100 features
+//   4,197 -> 3,362; of 30 features, 16 blocks a CU, 3,576, two waves 3,690);
+//   fewer trees leave waves idle in their last turn (100 trees: 80 features
+//   467, four waves 488), unless LDS holds five blocks at most (120 trees,
+//   125 features: 1,294 -> 688).
+uint32_t Forest::pair_waves(uint64_t blocks, uint64_t block_bytes) const {
+    const uint64_t cus = (uint64_t)dev_.cu_count(), lds = 160ull * 1024;
+    auto resident = [&](uint64_t w) { return w * (lds / (block_bytes + (w > 1 ? w * kPairTreeBytes : 0))); };
+    uint64_t w = 1;
+    if (blocks <= 4 * cus) {
+        w = blocks <= cus ? 16 : blocks <= 2 * cus ? 8 : 4;
+    } else if (resident(1) < (n_trees_ >= 256 ? 16 : 6)) {
+        for (w = 2; w < 8 && resident(w) <= 12;) w *= 2;
+    }
+    w = std::min<uint64_t>(w, (n_trees_ + 15) / 16);
+    while (w > 1 && resident(w) == 0) w--;
+    return (uint32_t)w;
+}
+
+void Forest::predict_pairs(PredictArgs a, uint64_t block_bytes, bool nan) {
+    const uint64_t lds = 160ull * 1024, cus = (uint64_t)dev_.cu_count();
+    const uint64_t blocks = ((uint64_t)a.n + 63) / 64;
+    const uint32_t waves = pair_waves(blocks, block_bytes);
+    if (waves > 1) {
+        const uint64_t bytes = block_bytes + waves * kPairTreeBytes;
+        const uint64_t grid = std::min<uint64_t>(blocks, cus * (lds / bytes));
+        dev_.launch(nan ? "hbr_predict_pairs_shared_nan" : "hbr_predict_pairs_shared", dim3((uint32_t)grid),
+                    dim3(64 * waves), a, (uint32_t)bytes);
+        return;
+    }
+    const uint64_t grid = std::min<uint64_t>(blocks, cus * (lds / block_bytes));  // a wave a block
+    dev_.launch(nan ? "hbr_predict_pairs_nan" : "hbr_predict_pairs", dim3((uint32_t)grid), dim3(64), a,
+                (uint32_t)block_bytes);
+}
+
 void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float missing, float *out,
                             int32_t *leaf_out, const float *init) {
     if (n == 0) return;
@@ -331,9 +394,11 @@ void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float m
         a.pair_values = pair_values_.get();
         a.pair_orig = pair_orig_.get();
         a.pair_levels = pair_levels_;
-        const uint64_t grid = std::min<uint64_t>(blocks, (uint64_t)dev_.cu_count() * (lds_total / mirror_block));
-        dev_.launch(nan ? "hbr_predict_pairs_nan" : "hbr_predict_pairs", dim3((uint32_t)grid), dim3(64), a,
-                    (uint32_t)mirror_block);
+        a.pair_tree = pair_tree_.get();
+        a.pair_output = pair_output_.get();
+        a.pair_weight = pair_weight_.get();
+        a.pair_first = pair_first_.get();
+        predict_pairs(a, mirror_block, nan);
         return;
     }
     // the mirror arena, one level per step

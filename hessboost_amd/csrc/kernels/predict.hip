@@ -104,14 +104,14 @@ __device__ __forceinline__ float mirror_value(float v, float missing) {
 
 template <bool NT = false, bool MIRROR = false, bool MISSING_NAN = true>
 __device__ __forceinline__ void stage_rows(float *s_x, const float *src, uint32_t rows, uint32_t n_cols,
-                                           uint32_t lane, float missing = 0.0f) {
+                                           uint32_t lane, float missing = 0.0f, uint32_t step = kPredLanes) {
     if (MIRROR) s_x += kPredPitch;
     const uint32_t total = rows * n_cols;
     const uint32_t n4 = ((uintptr_t)src & 15u) == 0 ? total / 4 : 0;  // an unaligned caller pointer: scalar
     const float inv = 1.0f / (float)n_cols;
     const float4 *src4 = reinterpret_cast<const float4 *>(src);
 #pragma unroll 5
-    for (uint32_t i = lane; i < n4; i += kPredLanes) {
+    for (uint32_t i = lane; i < n4; i += step) {
         typedef float f4 __attribute__((ext_vector_type(4)));
         const f4 nv = NT ? __builtin_nontemporal_load(reinterpret_cast<const f4 *>(src4) + i) : f4{};
         const float4 v = NT ? float4{nv.x, nv.y, nv.z, nv.w} : src4[i];
@@ -130,7 +130,7 @@ __device__ __forceinline__ void stage_rows(float *s_x, const float *src, uint32_
             }
         }
     }
-    for (uint32_t e = n4 * 4 + lane; e < total; e += kPredLanes) {
+    for (uint32_t e = n4 * 4 + lane; e < total; e += step) {
         const uint32_t rl = e / n_cols;
         const float v = src[e];
         s_x[(e - rl * n_cols) * kPredPitch + rl] = MIRROR ? mirror_value<MISSING_NAN>(v, missing) : v;
@@ -566,15 +566,65 @@ __device__ __forceinline__ uint32_t pair_step(uint32_t lane4, uint4 rec, uint32_
     return double_add(double_add(pos, go), go_c);
 }
 
-// Complete trees walked two levels per record (PredictArgs::pairs), LEVELS
-// records deep: rows resident in LDS as in hbr_predict_mirror (one 64-row
-// block per one-wave workgroup, slot 0 NaN), CH trees in flight per lane.
-// The root record and the tree's weight are the same for every lane (scalar
-// loads); a deeper record is read at the tree's level base, a uniform
-// address, plus the lane's 32-bit byte offset, and so is the leaf's value:
-// a tree costs the texture path one load per level below the root's two and
-// one for the leaf. The levels are unrolled so that a chain's next load can
-// issue as soon as its own step is done.
+// The leaf values and positions of the CH trees from t0 (the last group
+// repeats its last tree), LEVELS records deep. The root record and the
+// tree's weight are the same for every lane (scalar loads); a deeper record
+// is read at the tree's level base, a uniform address, plus the lane's
+// 32-bit byte offset, and so is the leaf's value: a tree costs the texture
+// path one load per level below the root's two and one for the leaf. The
+// levels are unrolled so that a chain's next load can issue as soon as its
+// own step is done.
+template <int CH, int LEVELS>
+__device__ __forceinline__ void walk_pairs(const PredictArgs &a, uint32_t lane4, uint32_t t0, uint32_t (&pos)[CH],
+                                           uint32_t (&leaf)[CH]) {
+    constexpr uint32_t per_tree = ((1u << (2 * LEVELS)) - 1u) / 3u;  // records
+    constexpr uint32_t leaves = 1u << (2 * LEVELS);
+    // the group's trees from one base: tree t0 + k at k' = min(k, last)
+    const uint32_t last = a.n_trees - 1 - t0;
+    const char *group = reinterpret_cast<const char *>(a.pairs + (size_t)t0 * per_tree);
+    const char *group_vals = reinterpret_cast<const char *>(a.pair_values + (size_t)t0 * leaves);
+#pragma unroll
+    for (int k = 0; k < CH; k++) {
+        const PairRecord rec = uniform_load(a.pairs, (size_t)(t0 + min((uint32_t)k, last)) * per_tree);
+        pos[k] = pair_step(lane4, make_uint4(rec.t_node, rec.t_first, rec.t_second, rec.s), 0u);
+    }
+#pragma unroll
+    for (int l = 1; l < LEVELS; l++) {
+        const uint32_t base = ((1u << (2 * l)) - 1u) / 3u;  // first record of the level
+        uint4 rec[CH];
+#pragma unroll
+        for (int k = 0; k < CH; k++) {
+            const uint32_t at = (min((uint32_t)k, last) * per_tree + base) * 16u + (pos[k] << 4);
+            rec[k] = *reinterpret_cast<const uint4 *>(group + at);
+        }
+#pragma unroll
+        for (int k = 0; k < CH; k++) pos[k] = pair_step(lane4, rec[k], pos[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < CH; k++)
+        leaf[k] = *reinterpret_cast<const uint32_t *>(group_vals + min((uint32_t)k, last) * leaves * 4u + (pos[k] << 2));
+}
+
+// A row's margins as the trees come, grouped by output (PredictArgs::pair_tree):
+// the running output's margin in a register, stored when the output changes.
+// (A read and write of the margin in memory per tree, the outputs taking
+// turns, waited for the store before it: 200k x 50 rows, 1,000 trees of 10
+// outputs took 1,530 us.)
+struct OutputSum {
+    float acc;
+    uint32_t cur;
+};
+
+__device__ __forceinline__ void next_output(const PredictArgs &a, uint32_t r, float *out, OutputSum &s, uint32_t o) {
+    if (o == s.cur) return;  // uniform
+    out[s.cur] = s.acc;
+    s.cur = o;
+    s.acc = start_margin(a, r, o);
+}
+
+// Complete trees walked two levels per record (PredictArgs::pairs): rows
+// resident in LDS as in hbr_predict_mirror (one 64-row block per one-wave
+// workgroup, slot 0 NaN), CH trees in flight per lane.
 // ONE: one output and no leaf indices (the margins alone, added in
 // registers).
 template <bool MISSING_NAN, int CH, int LEVELS, bool ONE>
@@ -583,7 +633,6 @@ __device__ __forceinline__ void predict_pairs(const PredictArgs &a) {
     const uint32_t lane = lane_id();
     const uint32_t lane4 = lane * 4u;
     s_rows[lane] = __builtin_nanf("");
-    constexpr uint32_t per_tree = ((1u << (2 * LEVELS)) - 1u) / 3u;  // records
     constexpr uint32_t leaves = 1u << (2 * LEVELS);
     const uint32_t n_blocks = (a.n + kPredLanes - 1) / kPredLanes;
     for (uint32_t blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
@@ -599,93 +648,143 @@ __device__ __forceinline__ void predict_pairs(const PredictArgs &a) {
         if (lane >= rows) continue;
         const uint32_t r = r0 + lane;
         float *out = a.out + (size_t)r * a.n_outputs;
-        if (a.n_outputs != 1)
+        if (!ONE)
             for (uint32_t o = 0; o < a.n_outputs; o++) out[o] = start_margin(a, r, o);
-        float acc = start_margin(a, r, 0);
+        OutputSum sum{0.0f, ONE ? 0u : uniform_load(a.pair_output, 0)};
+        sum.acc = start_margin(a, r, sum.cur);
         for (uint32_t t0 = 0; t0 < a.n_trees; t0 += CH) {
-            // the group's trees from one base: tree t0 + k at k' = min(k,
-            // last) trees past it (the last group repeats its last tree)
-            const uint32_t last = a.n_trees - 1 - t0;
-            const char *group = reinterpret_cast<const char *>(a.pairs + (size_t)t0 * per_tree);
-            const char *group_vals = reinterpret_cast<const char *>(a.pair_values + (size_t)t0 * leaves);
-            uint32_t pos[CH];
-#pragma unroll
-            for (int k = 0; k < CH; k++) {
-                const PairRecord rec = uniform_load(a.pairs, (size_t)(t0 + min((uint32_t)k, last)) * per_tree);
-                pos[k] = pair_step(lane4, make_uint4(rec.t_node, rec.t_first, rec.t_second, rec.s), 0u);
-            }
-#pragma unroll
-            for (int l = 1; l < LEVELS; l++) {
-                const uint32_t base = ((1u << (2 * l)) - 1u) / 3u;  // first record of the level
-                uint4 rec[CH];
-#pragma unroll
-                for (int k = 0; k < CH; k++) {
-                    const uint32_t at = (min((uint32_t)k, last) * per_tree + base) * 16u + (pos[k] << 4);
-                    rec[k] = *reinterpret_cast<const uint4 *>(group + at);
-                }
-#pragma unroll
-                for (int k = 0; k < CH; k++) pos[k] = pair_step(lane4, rec[k], pos[k]);
-            }
-            uint32_t leaf[CH];
-#pragma unroll
-            for (int k = 0; k < CH; k++)
-                leaf[k] = *reinterpret_cast<const uint32_t *>(group_vals + min((uint32_t)k, last) * leaves * 4u +
-                                                              (pos[k] << 2));
+            uint32_t pos[CH], leaf[CH];
+            walk_pairs<CH, LEVELS>(a, lane4, t0, pos, leaf);
 #pragma unroll
             for (int k = 0; k < CH; k++) {
                 const uint32_t t = t0 + (uint32_t)k;
                 if (t < a.n_trees) {
-                    const float contrib = uniform_load(a.tree_weight, t) * __uint_as_float(leaf[k]);
+                    const float contrib = uniform_load(a.pair_weight, t) * __uint_as_float(leaf[k]);
                     if (ONE) {
-                        acc = acc + contrib;
+                        sum.acc = sum.acc + contrib;
                         continue;
                     }
-                    if (a.leaf_out) a.leaf_out[(size_t)r * a.n_trees + t] = a.pair_orig[(size_t)t * leaves + pos[k]];
-                    if (a.n_outputs == 1) {
-                        acc = acc + contrib;
-                    } else {
-                        float *o = out + a.tree_output[t];
-                        *o = *o + contrib;
-                    }
+                    if (a.leaf_out)
+                        a.leaf_out[(size_t)r * a.n_trees + uniform_load(a.pair_tree, t)] =
+                            a.pair_orig[(size_t)t * leaves + pos[k]];
+                    next_output(a, r, out, sum, uniform_load(a.pair_output, t));
+                    sum.acc = sum.acc + contrib;
                 }
             }
         }
-        if (a.n_outputs == 1) out[0] = acc;
+        out[sum.cur] = sum.acc;
     }
 }
 
-template <bool MISSING_NAN, bool ONE>
+// The same walk with a 64-row block shared by a workgroup's waves, for
+// batches of too few blocks to fill the chip with a wave each: a wave walks
+// CH of every blockDim / 64 x CH trees and leaves their weighted leaf values
+// in LDS, and the first wave adds them to the margins in tree order (the
+// f32 additions of the one-wave walk, one by one).
+template <bool MISSING_NAN, int CH, int LEVELS, bool ONE>
+__device__ __forceinline__ void predict_pairs_shared(const PredictArgs &a) {
+    extern __shared__ float s_rows[];  // (n_cols + 1) * kPredPitch, then the trees' values [trees][kPredPitch]
+    float *s_val = s_rows + (size_t)(a.n_cols + 1) * kPredPitch;
+    const uint32_t lane = lane_id(), wave = threadIdx.x / kPredLanes;
+    const uint32_t lane4 = lane * 4u;
+    const uint32_t at_once = blockDim.x / kPredLanes * CH;
+    if (wave == 0) s_rows[lane] = __builtin_nanf("");
+    constexpr uint32_t leaves = 1u << (2 * LEVELS);
+    const uint32_t n_blocks = (a.n + kPredLanes - 1) / kPredLanes;
+    for (uint32_t blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
+        const uint32_t r0 = blk * kPredLanes;
+        const uint32_t rows = min(kPredLanes, a.n - r0);
+        const uint32_t r = r0 + min(lane, rows - 1);  // lanes past the rows walk what LDS holds, and store nothing
+        float *out = a.out + (size_t)r * a.n_outputs;
+        stage_rows<true, true, MISSING_NAN>(s_rows, a.x + (size_t)r0 * a.n_cols, rows, a.n_cols, threadIdx.x, a.missing,
+                                            blockDim.x);
+        OutputSum sum{0.0f, 0u};
+        const bool adds = wave == 0 && lane < rows;
+        if (adds) {
+            if (!ONE) {
+                for (uint32_t o = 0; o < a.n_outputs; o++) out[o] = start_margin(a, r, o);
+                sum.cur = uniform_load(a.pair_output, 0);
+            }
+            sum.acc = start_margin(a, r, sum.cur);
+        }
+        __syncthreads();
+        for (uint32_t c0 = 0; c0 < a.n_trees; c0 += at_once) {
+            const uint32_t t0 = c0 + wave * CH;
+            if (t0 < a.n_trees) {
+                uint32_t pos[CH], leaf[CH];
+                walk_pairs<CH, LEVELS>(a, lane4, t0, pos, leaf);
+#pragma unroll
+                for (int k = 0; k < CH; k++) {
+                    const uint32_t t = t0 + (uint32_t)k;
+                    if (t < a.n_trees) {
+                        s_val[(wave * CH + (uint32_t)k) * kPredPitch + lane] =
+                            uniform_load(a.pair_weight, t) * __uint_as_float(leaf[k]);
+                        if (!ONE && a.leaf_out && lane < rows)
+                            a.leaf_out[(size_t)r * a.n_trees + uniform_load(a.pair_tree, t)] =
+                                a.pair_orig[(size_t)t * leaves + pos[k]];
+                    }
+                }
+            }
+            __syncthreads();
+            if (adds) {
+                const uint32_t trees = min(at_once, a.n_trees - c0);
+                for (uint32_t k = 0; k < trees;) {
+                    // the output's trees among these
+                    const uint32_t end = ONE ? trees : min(trees, uniform_load(a.pair_first, sum.cur + 1) - c0);
+#pragma unroll 8
+                    for (; k < end; k++) sum.acc = sum.acc + s_val[k * kPredPitch + lane];
+                    if (!ONE && k < trees) next_output(a, r, out, sum, uniform_load(a.pair_output, c0 + k));
+                }
+            }
+            __syncthreads();  // the next trees' values, or the next block's rows
+        }
+        if (adds) out[sum.cur] = sum.acc;
+    }
+}
+
+template <bool MISSING_NAN, bool ONE, bool SHARED, int LEVELS>
+__device__ __forceinline__ void predict_pairs_walk(const PredictArgs &a) {
+    if constexpr (SHARED) predict_pairs_shared<MISSING_NAN, 16, LEVELS, ONE>(a);
+    else predict_pairs<MISSING_NAN, 16, LEVELS, ONE>(a);
+}
+
+template <bool MISSING_NAN, bool ONE, bool SHARED>
 __device__ __forceinline__ void predict_pairs_levels(const PredictArgs &a) {
     switch (a.pair_levels) {
-    case 1: predict_pairs<MISSING_NAN, 16, 1, ONE>(a); break;
-    case 2: predict_pairs<MISSING_NAN, 16, 2, ONE>(a); break;
-    case 3: predict_pairs<MISSING_NAN, 16, 3, ONE>(a); break;
-    case 4: predict_pairs<MISSING_NAN, 16, 4, ONE>(a); break;
-    case 5: predict_pairs<MISSING_NAN, 16, 5, ONE>(a); break;
-    case 6: predict_pairs<MISSING_NAN, 16, 6, ONE>(a); break;
+    case 1: predict_pairs_walk<MISSING_NAN, ONE, SHARED, 1>(a); break;
+    case 2: predict_pairs_walk<MISSING_NAN, ONE, SHARED, 2>(a); break;
+    case 3: predict_pairs_walk<MISSING_NAN, ONE, SHARED, 3>(a); break;
+    case 4: predict_pairs_walk<MISSING_NAN, ONE, SHARED, 4>(a); break;
+    case 5: predict_pairs_walk<MISSING_NAN, ONE, SHARED, 5>(a); break;
+    case 6: predict_pairs_walk<MISSING_NAN, ONE, SHARED, 6>(a); break;
     default: break;  // the host builds pair forests of depth 12 at most
     }
 }
 
-template <bool MISSING_NAN>
+template <bool MISSING_NAN, bool SHARED>
 __device__ __forceinline__ void predict_pairs_dispatch(const PredictArgs &a) {
     if (a.n_outputs == 1 && !a.leaf_out)
-        predict_pairs_levels<MISSING_NAN, true>(a);
+        predict_pairs_levels<MISSING_NAN, true, SHARED>(a);
     else
-        predict_pairs_levels<MISSING_NAN, false>(a);
+        predict_pairs_levels<MISSING_NAN, false, SHARED>(a);
 }
 
 // The occupancy is the LDS row blocks' (a few waves per SIMD): the walk may
 // keep its sixteen chains' records in registers.
 extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void hbr_predict_pairs_nan(
     PredictArgs a) {
-    predict_pairs_dispatch<true>(a);
+    predict_pairs_dispatch<true, false>(a);
 }
 extern "C" __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void hbr_predict_pairs(
     PredictArgs a) {
-    predict_pairs_dispatch<false>(a);
+    predict_pairs_dispatch<false, false>(a);
 }
-
+extern "C" __global__ __launch_bounds__(1024) void hbr_predict_pairs_shared_nan(PredictArgs a) {
+    predict_pairs_dispatch<true, true>(a);
+}
+extern "C" __global__ __launch_bounds__(1024) void hbr_predict_pairs_shared(PredictArgs a) {
+    predict_pairs_dispatch<false, true>(a);
+}
 // ---- evaluation sets --------------------------------------------------------
 //
 // A finished tree added into an evaluation set's margins as the host's
