@@ -23,9 +23,7 @@ public:
     // margins) may be null: the base scores.
     void predict_device(const float *x, uint64_t n, uint64_t n_cols, float missing, float *out, int32_t *leaf_out,
                         const float *init = nullptr);
-    // The same with x, init and out in host memory (pageable): beyond two
-    // chunks of rows, through Device::host_rows (the walk runs on each chunk
-    // while the next is staged and copied).
+    // The same with x, init and out in host memory (pageable).
     void predict_host(const float *x, uint64_t n, uint64_t n_cols, float missing, float *out, const float *init);
 
 private:
@@ -47,6 +45,9 @@ private:
     uint32_t chunk_cap_ = 0, n_chunks_ = 0;
     DBuf<uint32_t> chunk_tree_, chunk_node_;
     void plan_chunks(uint32_t cap);
+    // predict_host's buffers
+    PinnedBuf direct_;
+    DBuf<float> host_x_, host_out_, host_init_;
     DBuf<int32_t> orig_;
     DBuf<float> weight_, base_;
     // the mirror arena (absent with categorical splits, a non-finite

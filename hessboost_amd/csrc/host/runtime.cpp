@@ -181,7 +181,7 @@ void Device::reset_stats() {
 // is the processors', whatever the process last set for its own parallel
 // regions.
 static void copy_threads(void *dst, const void *src, uint64_t bytes) {
-    constexpr uint64_t kPiece = 4ull << 20;
+    constexpr uint64_t kPiece = 256ull << 10;
     const int64_t pieces = (int64_t)((bytes + kPiece - 1) / kPiece);
     const int threads = std::max(1, std::min(32, omp_get_num_procs()));
 #pragma omp parallel for schedule(static) num_threads(threads)

@@ -47,3 +47,22 @@ def test_shared_blocks_equal_the_mirror_walk(monkeypatch, n, trees, depth, f, ou
     for got, want in zip(pairs, all_of()):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
+
+
+# host rows read in place (up to 256 KiB), in one copy (up to 1 MiB), in chunks
+@pytest.mark.parametrize("n", [1, 700, 1_250, 2_180, 2_200, 8_700, 8_800, 20_011])
+@pytest.mark.parametrize("outputs", [1, 3])
+def test_host_rows_of_every_size_equal_device_rows(n, outputs):
+    rng = np.random.default_rng(n + outputs)
+    f = 30
+    forest = hb.Forest(_forest(rng, 40, 5, f, outputs), outputs)
+    x = rng.standard_normal((n, f), dtype=np.float32)
+    x[rng.random(x.shape) < 0.05] = np.nan
+    dx, dout = hb.DeviceBuffer(x.nbytes), hb.DeviceBuffer(4 * n * outputs)
+    dx.upload(x)
+    forest.predict_margin_device(dx.ptr, n, f, dout.ptr)
+    want = dout.download(np.float32, n * outputs)
+    init = np.tile(forest.arrs["base_score"], (n, 1))
+    for _ in range(2):
+        assert np.array_equal(forest.predict_margin(x).view(np.uint32), want.view(np.uint32))
+        assert np.array_equal(forest.predict_margin(x, init_margins=init).view(np.uint32), want.view(np.uint32))
