@@ -623,6 +623,8 @@ struct ScanArgs {
     uint32_t guard;          // 1: bound each candidate's error and flag near ties (kScanNearTie)
     uint32_t *cat_sets;
     uint32_t *best_sets;
+    uint32_t subtract;       // 1 (both children of every split): hbr_scan_sparse takes the siblings first
+    uint32_t pad;
 };
 
 // A level's reduce and search in one launch (hbr_reduce_scan).

@@ -1459,10 +1459,14 @@ void Engine::launch_scan(const ScanNode *nodes_dev, uint32_t n, const PartSplit 
         a.cat_sets = d_cat_sets_.get();
         a.best_sets = best_sets_dev;
     }
+    // the dense histograms turn each parent into the sibling as they finish;
+    // a sparse level's search does
+    const bool sparse = !dense_u8_ && !dense16_;
+    a.subtract = sparse && splits_dev ? 1u : 0u;
     if (grow)  // both children of each split; launch_hist left the reduce to it
         dev_.launch("hbr_reduce_scan", dim3(n_cols_, n / 2), dim3(512), ReduceScanArgs{reduce_args_, a});
     else
-        dev_.launch("hbr_scan_features", dim3(ceil_div(pairs, 4)), dim3(256), a);
+        dev_.launch(sparse ? "hbr_scan_sparse" : "hbr_scan_features", dim3(ceil_div(pairs, 4)), dim3(256), a);
     if (n_cat_) dev_.launch("hbr_scan_categorical", dim3(n * n_cat_), dim3(64), a);
     dev_.launch("hbr_scan_merge", dim3(n), dim3(256), a);
 }
@@ -1650,10 +1654,6 @@ std::vector<LevelChild> Engine::level(const std::vector<LevelSplit> &splits, boo
 
     if (!terminal) {
         launch_hist(reinterpret_cast<const HistNode *>(dev_in + o_hnodes), P, &hn, splits_dev, pout_dev);
-        if (!dense_u8_ && !dense16_) {  // the dense kernels turn each parent into the sibling as they finish
-            SubArgs sub{splits_dev, P, hist_.get(), total_bins_};
-            dev_.launch("hbr_subtract", dim3(std::min<uint32_t>(ceil_div(total_bins_, 256), 64), P), dim3(256), sub);
-        }
         launch_scan(reinterpret_cast<const ScanNode *>(dev_in + o_snodes), 2 * P, splits_dev, pout_dev,
                     reinterpret_cast<ScanBest *>(dev_out + o_best), nullptr,
                     n_cat_ ? reinterpret_cast<uint32_t *>(dev_out + o_sets) : nullptr);

@@ -257,8 +257,27 @@ __device__ __forceinline__ float up32(double x) {
     return f;
 }
 
-template <uint32_t BPL, bool GUARD>
-__device__ __forceinline__ void scan_feature(const ScanArgs &a, uint32_t node, uint32_t f, ScanBest *out) {
+// Candidates of one wave's chunk, packed: the sums below (or from) a bin, and
+// the bin.
+struct ScanList {
+    int64_t g[256], h[256];
+    uint32_t bin[256];
+};
+
+// SPARSE: candidates that repeat an earlier one's sums are left out. The
+// prefix at an empty bin is the bin's before it, the suffix from one the next
+// bin's, and equal sums are the same score, of which the first candidate
+// wins. The kept ones of BPL > 1 are packed in LDS and taken a lane each: the
+// f64 scores are what the search costs, and a sparse node of few rows has few
+// bins that are not empty. With ScanArgs::subtract the wave of a child that is
+// not built takes its bins as the parent's less the built child's and stores
+// them in the parent's slot, which no other wave reads. A batch of best-first
+// splits over 100k x 1,000 sparse rows: 63 us and 18 for the subtraction, now
+// 46 together. Dense nodes fill their bins: packed, the search of 512 bins a
+// feature took 15.1 us, in registers 13.5.
+template <uint32_t BPL, bool GUARD, bool SPARSE>
+__device__ __forceinline__ void scan_feature(const ScanArgs &a, uint32_t node, uint32_t f, ScanBest *out,
+                                             ScanList *list) {
     const uint32_t lane = lane_id();
     const ScanNode nd = a.nodes[node];
     const uint32_t fs = a.feature_offset[f], nb = a.feature_offset[f + 1] - fs;
@@ -273,7 +292,13 @@ __device__ __forceinline__ void scan_feature(const ScanArgs &a, uint32_t node, u
     Rivals riv;
     riv.init();
     Bound bound{0.0, 0.0};
-    const QBin *h = a.hist + (size_t)node_slot(a, nd) * a.total_bins + fs;
+    const uint32_t slot = node_slot(a, nd);
+    const QBin *h = a.hist + (size_t)slot * a.total_bins + fs;
+    const QBin *built = nullptr;  // the built child's bins, to be taken from h first
+    if (SPARSE && a.subtract) {
+        const uint32_t fresh = a.splits[nd.split].fresh_slot;
+        if (slot != fresh) built = a.hist + (size_t)fresh * a.total_bins + fs;
+    }
     const bool dev_root = (nd.pad & kScanDeviceRoot) != 0;
     const uint32_t cls = nd.pad >> kScanClassShift;
     QBin *root_total = a.root_total + cls;
@@ -307,82 +332,91 @@ __device__ __forceinline__ void scan_feature(const ScanArgs &a, uint32_t node, u
         if (GUARD)
             bound = node_bound(node_rows(a, nd), eg, eh, __uint_as_float(a.scale[cls].max_g_bits),
                                __uint_as_float(a.scale[cls].max_h_bits));
-        int64_t carry_g = 0, carry_h = 0;
-        // forward pass: bins <= b left, missing right
-        for (uint32_t c0 = 0; c0 < nb; c0 += kWave * BPL) {
-            const uint32_t b0 = c0 + BPL * lane;
-            int64_t sg[BPL], sh[BPL];
-            int64_t rg = 0, rh = 0;
-#pragma unroll
-            for (int k = 0; k < (int)BPL; k++) {
-                QBin v = (b0 + k < nb) ? h[b0 + k] : QBin{0, 0};
-                rg += v.g;
-                rh += v.h;
-                sg[k] = rg;
-                sh[k] = rh;
+        auto consider = [&](int64_t lg, int64_t lh, uint32_t idx, uint32_t backward) {
+            float loss;
+            if (GUARD) {
+                const Scored sc = score_guarded(dequant(lg, eg), dequant(lh, eh), dequant(tg - lg, eg),
+                                                dequant(th - lh, eh), a.reg, nd.lower, nd.upper, dir, root_gain, bound);
+                if (sc.ok) offer(best, nan_seen, sc.loss, idx, lg, lh, tg - lg, th - lh, backward, sc.err, sc.fragile);
+                if (sc.rival) riv.offer(up32((double)sc.loss + (double)sc.err), lg, lh);
+            } else if (score(dequant(lg, eg), dequant(lh, eh), dequant(tg - lg, eg), dequant(th - lh, eh), a.reg,
+                             nd.lower, nd.upper, dir, root_gain, &loss)) {
+                offer(best, nan_seen, loss, idx, lg, lh, tg - lg, th - lh, backward);
             }
-            const int64_t ig = wave_inclusive_scan(rg), ih = wave_inclusive_scan(rh);
-            const int64_t xg = carry_g + ig - rg, xh = carry_h + ih - rh;
-#pragma unroll
-            for (int k = 0; k < (int)BPL; k++) {
-                if (b0 + k >= nb) break;
-                const int64_t ag = xg + sg[k], ah = xh + sh[k];
-                float loss;
-                if (GUARD) {
-                    const Scored sc = score_guarded(dequant(ag, eg), dequant(ah, eh), dequant(tg - ag, eg),
-                                                    dequant(th - ah, eh), a.reg, nd.lower, nd.upper, dir, root_gain,
-                                                    bound);
-                    if (sc.ok) offer(best, nan_seen, sc.loss, b0 + k, ag, ah, tg - ag, th - ah, 0, sc.err, sc.fragile);
-                    if (sc.rival) riv.offer(up32((double)sc.loss + (double)sc.err), ag, ah);
-                } else if (score(dequant(ag, eg), dequant(ah, eh), dequant(tg - ag, eg), dequant(th - ah, eh), a.reg,
-                                 nd.lower, nd.upper, dir, root_gain, &loss)) {
-                    offer(best, nan_seen, loss, b0 + k, ag, ah, tg - ag, th - ah, 0);
-                }
-            }
-            carry_g += wave_broadcast(ig, kWave - 1);
-            carry_h += wave_broadcast(ih, kWave - 1);
-        }
-        // backward pass: bins >= b right, missing left; ends below every bin
-        if (!a.dense && (carry_g != tg || carry_h != th)) {
-            const int64_t fg = carry_g, fh = carry_h;
-            carry_g = carry_h = 0;
+        };
+        int64_t fg = 0, fh = 0;  // the bins' sum, after the forward pass
+        for (uint32_t backward = 0; backward < 2; backward++) {
+            // forward: bins <= b left, missing right. Backward: bins >= b
+            // right, missing left; ends below every bin.
+            if (backward && (a.dense || (fg == tg && fh == th))) break;
+            int64_t carry_g = 0, carry_h = 0;
             for (uint32_t c0 = 0; c0 < nb; c0 += kWave * BPL) {
                 const uint32_t b0 = c0 + BPL * lane;
-                int64_t eg_[BPL], eh_[BPL];  // exclusive prefix of each bin
+                QBin v[BPL];
                 int64_t rg = 0, rh = 0;
 #pragma unroll
-                for (int k = 0; k < (int)BPL; k++) {
-                    QBin v = (b0 + k < nb) ? h[b0 + k] : QBin{0, 0};
-                    eg_[k] = rg;
-                    eh_[k] = rh;
-                    rg += v.g;
-                    rh += v.h;
+                for (int k = 0; k < (int)BPL; k++) v[k] = b0 + k < nb ? h[b0 + k] : QBin{0, 0};
+                if (built && !backward) {
+                    QBin c[BPL];
+#pragma unroll
+                    for (int k = 0; k < (int)BPL; k++) c[k] = b0 + k < nb ? built[b0 + k] : QBin{0, 0};
+#pragma unroll
+                    for (int k = 0; k < (int)BPL; k++) {
+                        v[k].g -= c[k].g;
+                        v[k].h -= c[k].h;
+                        if (b0 + k < nb) const_cast<QBin *>(h)[b0 + k] = v[k];
+                    }
                 }
-                const int64_t ig = wave_inclusive_scan(rg), ih = wave_inclusive_scan(rh);
-                const int64_t xg = carry_g + ig - rg, xh = carry_h + ih - rh;
 #pragma unroll
                 for (int k = 0; k < (int)BPL; k++) {
-                    const uint32_t o = b0 + k;
-                    if (o >= nb) break;
-                    const int64_t sgv = fg - (xg + eg_[k]), shv = fh - (xh + eh_[k]);  // suffix from bin o
-                    float loss;
-                    if (GUARD) {
-                        const Scored sc = score_guarded(dequant(tg - sgv, eg), dequant(th - shv, eh), dequant(sgv, eg),
-                                                        dequant(shv, eh), a.reg, nd.lower, nd.upper, dir, root_gain,
-                                                        bound);
-                        if (sc.ok)
-                            offer(best, nan_seen, sc.loss, nb + (nb - 1 - o), tg - sgv, th - shv, sgv, shv, 1, sc.err,
-                                  sc.fragile);
-                        if (sc.rival) riv.offer(up32((double)sc.loss + (double)sc.err), tg - sgv, th - shv);
-                    } else if (score(dequant(tg - sgv, eg), dequant(th - shv, eh), dequant(sgv, eg),
-                                     dequant(shv, eh), a.reg, nd.lower, nd.upper, dir, root_gain, &loss)) {
-                        offer(best, nan_seen, loss, nb + (nb - 1 - o), tg - sgv, th - shv, sgv, shv, 1);
+                    rg += v[k].g;
+                    rh += v[k].h;
+                }
+                const int64_t ig = wave_inclusive_scan(rg), ih = wave_inclusive_scan(rh);
+                int64_t ag = carry_g + ig - rg, ah = carry_h + ih - rh;
+                uint32_t kept = 0;
+#pragma unroll
+                for (int k = 0; k < (int)BPL; k++) {
+                    const uint32_t b = b0 + k;
+                    const bool keep = b < nb && (!SPARSE || (v[k].g | v[k].h) != 0 || b == (backward ? nb - 1 : 0u));
+                    // the left child's sums: the prefix, or all but the suffix from b
+                    int64_t lg = tg - (fg - ag), lh = th - (fh - ah);
+                    ag += v[k].g;
+                    ah += v[k].h;
+                    if (!backward) {
+                        lg = ag;
+                        lh = ah;
                     }
+                    if (BPL == 1 || !SPARSE) {
+                        if (keep) consider(lg, lh, backward ? nb + (nb - 1 - b) : b, backward);
+                        continue;
+                    }
+                    const uint64_t m = __ballot(keep);
+                    if (keep) {
+                        const uint32_t at = kept + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                        list->g[at] = lg;
+                        list->h[at] = lh;
+                        list->bin[at] = b;
+                    }
+                    kept += (uint32_t)__popcll(m);
+                }
+                if (BPL > 1 && SPARSE) {  // the wave's own list: its LDS accesses are in order
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    for (uint32_t e = lane; e < kept; e += kWave) {
+                        const uint32_t b = list->bin[e];
+                        consider(list->g[e], list->h[e], backward ? nb + (nb - 1 - b) : b, backward);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 }
                 carry_g += wave_broadcast(ig, kWave - 1);
                 carry_h += wave_broadcast(ih, kWave - 1);
             }
+            fg = carry_g;
+            fh = carry_h;
         }
+    } else if (built) {
+        for (uint32_t b = lane; b < nb; b += kWave)
+            const_cast<QBin *>(h)[b] = QBin{h[b].g - built[b].g, h[b].h - built[b].h};
     }
     // wave arg-best: highest loss, then lowest candidate index
     float bl = best.loss;
@@ -434,22 +468,32 @@ __device__ __forceinline__ void scan_feature(const ScanArgs &a, uint32_t node, u
     }
 }
 
-extern "C" __global__ __launch_bounds__(256) void hbr_scan_features(ScanArgs a) {
+template <bool SPARSE>
+__device__ __forceinline__ void scan_features(const ScanArgs &a, ScanList *lists) {
     const uint32_t wave = threadIdx.x / kWave;
     const uint32_t pair = blockIdx.x * (blockDim.x / kWave) + wave;
     if (pair >= scan_nodes(a) * a.n_features) return;  // uniform per wave
-    const uint32_t f = pair % a.n_features;
+    const uint32_t node = pair / a.n_features, f = pair % a.n_features;
     const bool narrow = a.feature_offset[f + 1] - a.feature_offset[f] <= kWave;  // uniform per wave
+    ScanBest *out = a.per_feature + pair;
+    ScanList *list = SPARSE ? lists + wave : nullptr;
     if (a.guard) {
-        if (narrow)
-            scan_feature<1, true>(a, pair / a.n_features, f, a.per_feature + pair);
-        else
-            scan_feature<4, true>(a, pair / a.n_features, f, a.per_feature + pair);
+        if (narrow) scan_feature<1, true, SPARSE>(a, node, f, out, list);
+        else scan_feature<4, true, SPARSE>(a, node, f, out, list);
     } else if (narrow) {
-        scan_feature<1, false>(a, pair / a.n_features, f, a.per_feature + pair);
+        scan_feature<1, false, SPARSE>(a, node, f, out, list);
     } else {
-        scan_feature<4, false>(a, pair / a.n_features, f, a.per_feature + pair);
+        scan_feature<4, false, SPARSE>(a, node, f, out, list);
     }
+}
+
+extern "C" __global__ __launch_bounds__(256) void hbr_scan_features(ScanArgs a) { scan_features<false>(a, nullptr); }
+
+// For an index of sparse rows; four waves a SIMD (128 registers) instead of
+// three (131) 46 us instead of 52, five would spill.
+extern "C" __global__ __launch_bounds__(256, 4) void hbr_scan_sparse(ScanArgs a) {
+    __shared__ ScanList s_list[256 / kWave];
+    scan_features<true>(a, s_list);
 }
 
 // hbr_hist_reduce and hbr_scan_features of a level's splits in one launch,

@@ -154,3 +154,30 @@ def test_best_first_trees_split_ahead_match_the_oracle(sparse, leaves, depth):
     compare_trees(t.trees(), ref.trees())
     assert np.max(np.abs(t.margins() - ref.margins().reshape(-1))) <= 1e-5
     assert engine.counters()["near_ties"] - before["near_ties"] <= sum(len(k["left"]) for k in t.trees())
+
+
+# sparse rows: most bins of a node empty (few rows) and none (many), features
+# of one bin, of at most 64, of up to 256 and of more (several chunks a pass)
+@pytest.mark.parametrize("n", [40, 3_000, 12_000])
+@pytest.mark.parametrize("bins", [20, 256, 700])
+@pytest.mark.parametrize("lossguide", [False, True])
+def test_sparse_search_and_siblings_match_the_oracle(n, bins, lossguide):
+    from oracle import oracle as O
+    from tests.test_gpu_train import compare_trees
+
+    rng = np.random.default_rng(n + bins)
+    f = 260  # more than masked rows take
+    x = rng.standard_normal((n, f)).astype(np.float32)
+    x[rng.random(x.shape) < 0.7] = np.nan
+    x[:, 3] = np.where(np.isnan(x[:, 3]), np.nan, 2.0)  # one bin
+    x[:, 4] = np.round(x[:, 4] * 3)
+    y = np.nan_to_num(x[:, 0]) - np.nan_to_num(x[:, 1]) * np.nan_to_num(x[:, 4]) + 0.5 * np.isnan(x[:, 3])
+    y = (y + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    grow = dict(max_depth=0, max_leaves=30) if lossguide else dict(max_depth=6)
+    params = dict(grow, max_bin=bins, eta=0.3, min_child_weight=2.0, grow_policy="lossguide" if lossguide else "depthwise")
+    more = dict(grow_policy=O.GROW_LOSSGUIDE) if lossguide else {}
+    ref = O.Model(O.Dataset(x, max_bin=bins), y, O.params(min_child_weight=2.0, **grow, **more), 2)
+    trees, margins, launches = _fit(x, y, params, 2)
+    assert launches.get("hbr_scan_sparse", 0) > 0 and "hbr_subtract" not in launches
+    compare_trees(trees, ref.trees())
+    assert np.max(np.abs(margins - ref.margins().reshape(-1))) <= 1e-5  # f32 sums of two leaves each
