@@ -817,6 +817,7 @@ struct WalkArgs {
     // go to output + c.
     uint32_t n_trees;
     uint32_t tree_bytes;
+    const uint16_t *bins16;      // hbr_walk_leaves16: rows of u16 bins [n][stride], instead of bins8
 };
 // Node tables of all the trees of one batched walk, in LDS.
 constexpr uint32_t kBatchWalkNodes = 2048;

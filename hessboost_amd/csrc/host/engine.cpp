@@ -1303,11 +1303,13 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     if (n == 0) return;
     root_partials_ = 0;  // the partials are reused below
     if (!level_pairs_ && !pairs_staged()) fail(kInvalid, "histograms: no gradients staged");
-    if (!dense_u8_ && grow) fail(kInvalid, "histograms: device-counted levels need the dense kernels");
+    if (!dense_u8_ && !dense16_ && grow) fail(kInvalid, "histograms: device-counted levels need the dense kernels");
     const bool wide = dense16_;  // u16 rows
     const uint32_t fg = wide ? fg16_ : masked_ ? 32u : hist_features_per_group;  // masked rows: fg32 groups
     const uint32_t group_bins = wide ? kWideLdsBins / fg16_ : 256u;
     const bool dense = dense_u8_ || wide;
+    // a device-grown level's partials of u8 rows are summed by its search
+    const bool reduce_in_scan = grow && dense_u8_;
     // dense: feature groups of fg features; CSR: ranges of kCsrGroupBins
     // global bins (every range of every tile is written: no slot zeroing)
     const uint32_t groups = dense ? ceil_div(n_cols_, fg) : ceil_div(total_bins_, kCsrGroupBins);
@@ -1329,7 +1331,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     p.tiles = d_htiles_.get();
     p.counts = d_hcounts_.get();
     p.min_cost = tile_cost(groups);
-    p.fuse_subtract = dense && !grow ? 1u : 0u;
+    p.fuse_subtract = dense && !reduce_in_scan ? 1u : 0u;
     p.grow = grow;
     dev_.launch("hbr_hist_plan", dim3(1), dim3(256), p);
 
@@ -1362,7 +1364,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     a.min_hess = row_pairs_min_hess_;
     a.bins16 = rows16_.get();
     a.stride16 = stride16_;
-    a.partials_only = grow ? 1u : 0u;
+    a.partials_only = reduce_in_scan ? 1u : 0u;
     static const char *const wide_kernels[] = {"hbr_hist_dense16_fg1", "hbr_hist_dense16_fg2", "hbr_hist_dense16_fg4",
                                                "hbr_hist_dense16_fg8", "hbr_hist_dense16_fg16"};
     const char *k = wide ? wide_kernels[__builtin_ctz(fg)] : !dense_u8_ ? "hbr_hist_csr" : dense8_kernel(fg);
@@ -1390,8 +1392,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
         r.grow = grow;
         r.group_bins = group_bins;
         r.quarters = group_bins / 64u;
-        // a device-grown level's partials are summed by its search
-        if (!grow) dev_.launch("hbr_hist_reduce", dim3(n_cols_ * r.quarters, n), dim3(1024), r);
+        if (!reduce_in_scan) dev_.launch("hbr_hist_reduce", dim3(n_cols_ * r.quarters, n), dim3(1024), r);
     }
 }
 
@@ -1463,7 +1464,7 @@ void Engine::launch_scan(const ScanNode *nodes_dev, uint32_t n, const PartSplit 
     // a sparse level's search does
     const bool sparse = !dense_u8_ && !dense16_;
     a.subtract = sparse && splits_dev ? 1u : 0u;
-    if (grow)  // both children of each split; launch_hist left the reduce to it
+    if (grow && dense_u8_)  // both children of each split; launch_hist left the reduce to it
         dev_.launch("hbr_reduce_scan", dim3(n_cols_, n / 2), dim3(512), ReduceScanArgs{reduce_args_, a});
     else
         dev_.launch(sparse ? "hbr_scan_sparse" : "hbr_scan_features", dim3(ceil_div(pairs, 4)), dim3(256), a);
@@ -1701,8 +1702,11 @@ std::vector<LevelChild> Engine::level(const std::vector<LevelSplit> &splits, boo
 // hold (2^level splits, every row in a split); the kernels read the real
 // counts from the device. The tree, its counts and the scale come back with
 // one copy after the last level.
+// Rows of u16 bins too, of an index with no missing cells: their levels cost
+// a copy and a wait each way on the host's path and three partition launches
+// (500k x 28 rows of 512 bins, depth 7: 107 us a level, decided here 80).
 bool Engine::can_grow_device(uint64_t max_depth, uint32_t n_trees) const {
-    if (!device_grow || !dense_u8_ || max_depth < 1 || max_depth > kMaxDeviceDepth || n_rows_ == 0) return false;
+    if (!device_grow || !(dense_u8_ || (dense16_ && cols16_.size())) || max_depth < 1 || max_depth > kMaxDeviceDepth || n_rows_ == 0) return false;
     if (n_cat_) return false;  // categorical splits are decided by the host
     if (n_trees < 1 || n_trees > kGrowMaxTrees || (uint64_t)n_trees * n_rows_ > UINT32_MAX) return false;
     const uint64_t slots = (uint64_t)n_trees << (max_depth - 1);
@@ -2049,10 +2053,10 @@ bool Engine::walk_device_trees(uint32_t first_output, uint32_t n_trees, uint32_t
 
 void Engine::walk_device_tree(uint32_t output, const hbr_device_loss *next_loss, uint32_t tree, uint32_t guard_first,
                               uint32_t guard_n) {
-    if (!dense_u8_) fail(kRefused, "walk: the index has no row-major u8 bins");
+    if (!dense_u8_ && !dense16_) fail(kRefused, "walk: the index has no row-major bins");
     if (output >= outputs_) fail(kInvalid, "walk: no such output");
     // the staged walk: 32-byte rows and trees whose nodes fit its LDS table
-    const bool staged = stride_ == 32 && last_depth_ <= 9;
+    const bool staged = dense_u8_ && stride_ == 32 && last_depth_ <= 9;
     if (next_loss && !staged) fail(kRefused, "walk: gradients need 32-byte rows and depth <= 9");
     hipStream_t s = dev_.stream();
     WalkArgs a{};
@@ -2061,8 +2065,9 @@ void Engine::walk_device_tree(uint32_t output, const hbr_device_loss *next_loss,
     a.tree = ring_nodes(last_ring_, tree, last_stride_);
     a.counts = &ring_header(last_ring_, tree, last_stride_)->counts;
     a.bins8 = rows8_.get();
+    a.bins16 = rows16_.get();
     a.margins = margins_.get();
-    a.stride = stride_;
+    a.stride = dense16_ ? stride16_ : stride_;
     a.n = (uint32_t)n_rows_;
     a.m_stride = outputs_;
     a.output = output;
@@ -2081,7 +2086,7 @@ void Engine::walk_device_tree(uint32_t output, const hbr_device_loss *next_loss,
             a.guard_n = guard_n;
             a.poison = poison_.get();
         }
-        dev_.launch(staged ? "hbr_walk_leaves32" : "hbr_walk_leaves", dim3(blocks), dim3(256), a);
+        dev_.launch(staged ? "hbr_walk_leaves32" : dense16_ ? "hbr_walk_leaves16" : "hbr_walk_leaves", dim3(blocks), dim3(256), a);
         return;
     }
     if (outputs_ != 1 || !labels_loaded_) fail(kInvalid, "walk: gradients need one output and labels");
@@ -2152,7 +2157,7 @@ void Engine::walk_device_tree(uint32_t output, const hbr_device_loss *next_loss,
 }
 
 void Engine::walk_device_tree_then_gradients(const hbr_device_loss &next_loss) {
-    if (!dense_u8_) fail(kRefused, "walk: the index has no row-major u8 bins");
+    if (!dense_u8_ && !dense16_) fail(kRefused, "walk: the index has no row-major bins");
     if (outputs_ != 1 || !labels_loaded_) fail(kInvalid, "walk: gradients need one output and labels");
     hipStream_t s = dev_.stream();
     if (!poison_.size()) {
@@ -2169,8 +2174,9 @@ void Engine::walk_device_tree_then_gradients(const hbr_device_loss &next_loss) {
     a.tree = ring_nodes(last_ring_, 0, last_stride_);
     a.counts = &ring_header(last_ring_, 0, last_stride_)->counts;
     a.bins8 = rows8_.get();
+    a.bins16 = rows16_.get();
     a.margins = margins_.get();
-    a.stride = stride_;
+    a.stride = dense16_ ? stride16_ : stride_;
     a.n = (uint32_t)n_rows_;
     a.m_stride = outputs_;
     a.output = 0;
@@ -2179,7 +2185,7 @@ void Engine::walk_device_tree_then_gradients(const hbr_device_loss &next_loss) {
     a.poison = poison_.get();
     const uint32_t blocks =
         std::min<uint32_t>(std::max<uint32_t>(1, ceil_div(n_rows_, 256)), (uint32_t)dev_.cu_count() * walk_blocks_per_cu);
-    dev_.launch("hbr_walk_leaves", dim3(blocks), dim3(256), a);
+    dev_.launch(dense16_ ? "hbr_walk_leaves16" : "hbr_walk_leaves", dim3(blocks), dim3(256), a);
     compute_gradients_async(next_loss, 0);
 }
 

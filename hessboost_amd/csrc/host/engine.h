@@ -237,9 +237,10 @@ public:
     // way by the softmax class scales [guard_first, guard_first + guard_n)
     // (the tree's class, or every class of a batched round).
     bool can_walk_device_tree(uint64_t max_depth) const {
-        return can_grow_device(max_depth) && stride_ == 32 && max_depth <= 9 && outputs_ == 1 && labels_loaded_;
+        return dense_u8_ && can_grow_device(max_depth) && stride_ == 32 && max_depth <= 9 && outputs_ == 1 &&
+               labels_loaded_;
     }
-    // The walk alone (no gradients): any dense u8 index, any output.
+    // The walk alone (no gradients): any dense u8 or u16 index, any output.
     bool can_route_device_tree(uint64_t max_depth) const { return can_grow_device(max_depth); }
     // The last queued device tree's leaves onto the margins of one output by
     // the walk of any row layout (wider rows, masked rows, deeper trees),

@@ -520,6 +520,7 @@ extern "C" __global__ __launch_bounds__(1024) void hbr_hist_csr(HistArgs a) { hi
 extern "C" __global__ __launch_bounds__(1024) void hbr_hist_reduce(ReduceArgs a) {
     __shared__ int64_t acc[2][16][64];
     const uint32_t f = blockIdx.x / a.quarters, quarter = blockIdx.x % a.quarters;
+    if (a.grow && blockIdx.y >= a.grow->n_splits) return;
     const HistNode nd = a.nodes[blockIdx.y];
     if (f >= a.n_cols || nd.n_tiles == 1) return;  // uniform across the workgroup
     const uint32_t lo = a.feature_offset[f], nb = a.feature_offset[f + 1] - lo;

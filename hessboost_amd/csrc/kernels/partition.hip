@@ -378,7 +378,8 @@ __device__ __forceinline__ void part_move(const PartArgs &a, const Bin *cols) {
 }
 
 extern "C" __global__ __launch_bounds__(1024, 8) void hbr_part_move(PartArgs a) {
-    if (a.missing) part_move<uint8_t, true>(a, a.cols8);
+    if (a.cols16) part_move<uint16_t, false>(a, a.cols16);  // (an index of u16 rows has no missing cells)
+    else if (a.missing) part_move<uint8_t, true>(a, a.cols8);
     else part_move<uint8_t, false>(a, a.cols8);
 }
 
@@ -430,11 +431,12 @@ __device__ __forceinline__ bool walk_skipped(const WalkArgs &a) {
     return bad != 0;
 }
 
-extern "C" __global__ __launch_bounds__(256) void hbr_walk_leaves(WalkArgs a) {
+template <typename Bin>
+__device__ __forceinline__ void walk_leaves(const WalkArgs &a, const Bin *bins) {
     if (walk_skipped(a)) return;
     const uint32_t n_nodes = walk_nodes(a);
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < a.n; r += gridDim.x * blockDim.x) {
-        const uint8_t *b = a.bins8 + (size_t)r * a.stride;
+        const Bin *b = bins + (size_t)r * a.stride;
         uint32_t nid = 0, left;
         uint32_t meta = node_meta(a, 0, &left);
         for (uint32_t step = 0; step < n_nodes && !(meta >> 31); step++) {
@@ -454,6 +456,9 @@ extern "C" __global__ __launch_bounds__(256) void hbr_walk_leaves(WalkArgs a) {
     }
 }
 
+extern "C" __global__ __launch_bounds__(256) void hbr_walk_leaves(WalkArgs a) { walk_leaves(a, a.bins8); }
+// Rows of u16 bins (stride in elements; no missing cells).
+extern "C" __global__ __launch_bounds__(256) void hbr_walk_leaves16(WalkArgs a) { walk_leaves(a, a.bins16); }
 
 
 // The walks for 32-byte rows and trees of at most kWalkLdsNodes nodes: the

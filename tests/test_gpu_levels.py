@@ -181,3 +181,21 @@ def test_sparse_search_and_siblings_match_the_oracle(n, bins, lossguide):
     assert launches.get("hbr_scan_sparse", 0) > 0 and "hbr_subtract" not in launches
     compare_trees(trees, ref.trees())
     assert np.max(np.abs(margins - ref.margins().reshape(-1))) <= 1e-5  # f32 sums of two leaves each
+
+
+# rows of u16 bins: each width of a feature group, one group and several, one
+# tile and many, class trees in a batch
+@pytest.mark.parametrize("n,f,bins,depth,classes", [
+    (1, 2, 300, 3, 0), (600, 17, 512, 1, 0), (5_000, 16, 300, 6, 0), (5_000, 5, 1000, 8, 0), (30_000, 33, 600, 5, 0),
+    (40_000, 3, 8000, 4, 0), (600_001, 2, 512, 4, 0), (20_000, 6, 400, 4, 3), (9_000, 4, 2000, 10, 0),
+])
+def test_device_growth_over_u16_bins_gives_the_host_levels_trees(monkeypatch, n, f, bins, depth, classes):
+    x, y = _data(n, f, 0.0, seed=n + bins, classes=classes)
+    params = {"objective": "multi:softprob" if classes else "binary:logistic", "max_depth": depth, "eta": 0.3,
+              "base_score": 0.5, "max_bin": bins}
+    if classes:
+        params["num_class"] = classes
+    device, host = _both(monkeypatch, x, y, params, 3)
+    if n > 1 and depth > 1:
+        assert device[2].get("hbr_part_move", 0) > 0 and device[2].get("hbr_walk_leaves16", 0) > 0
+    _same(device, host)
