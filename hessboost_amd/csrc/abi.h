@@ -959,9 +959,10 @@ struct alignas(8) CompactNode {
 // reads row l of every feature from bank l, whatever the feature.
 constexpr uint32_t kPredPitch = 64;
 
-// LDS a wave of the shared pair walk leaves its 16 trees' values of a 64-row
-// block in.
-constexpr uint32_t kPairTreeBytes = 16 * kPredPitch * 4;
+// Trees a wave of the pair walk keeps in flight, and the LDS in which a wave
+// of the shared walk leaves their values of a 64-row block.
+constexpr uint32_t kPairGroup = 16;
+constexpr uint32_t kPairTreeBytes = kPairGroup * kPredPitch * 4;
 
 // Two levels of a complete tree (PredictArgs::pairs).
 struct alignas(16) PairRecord {
@@ -1050,7 +1051,7 @@ struct PredictArgs {
     const uint32_t *pair_tree;     // n_trees: the caller's number of each tree
     const uint32_t *pair_output;   // n_trees, ascending
     const uint32_t *pair_first;    // n_outputs + 1: each output's first tree
-    const float *pair_weight;      // n_trees
+    const float *pair_weight;      // n_trees, padded to whole groups of kPairGroup
 };
 constexpr uint32_t kPredCategorical = 1u << 29;
 

@@ -231,17 +231,18 @@ void Forest::build_pairs(const hbr_forest_desc &fd) {
     pair_values_.upload(values.data(), values.size(), s);
     pair_orig_.resize(orig.size());
     pair_orig_.upload(orig.data(), orig.size(), s);
-    pair_tree_.resize(n_trees_);
-    pair_tree_.upload(order.data(), n_trees_, s);
-    pair_output_.resize(n_trees_);
-    pair_output_.upload(outputs.data(), n_trees_, s);
-    std::vector<uint32_t> first(n_outputs_ + 1);
+    // the trees' weights (padded to whole groups of the walk's trees),
+    // numbers and outputs, and each output's first tree: one upload
+    const size_t padded = (n_trees_ + kPairGroup - 1) / kPairGroup * kPairGroup;
+    std::vector<uint32_t> meta(padded + 2 * n_trees_ + n_outputs_ + 1, 0u);
+    std::memcpy(meta.data(), weights.data(), n_trees_ * sizeof(float));
+    std::copy(order.begin(), order.end(), meta.begin() + padded);
+    std::copy(outputs.begin(), outputs.end(), meta.begin() + padded + n_trees_);
     for (uint32_t o = 0; o <= n_outputs_; o++)
-        first[o] = (uint32_t)(std::lower_bound(outputs.begin(), outputs.end(), o) - outputs.begin());
-    pair_first_.resize(first.size());
-    pair_first_.upload(first.data(), first.size(), s);
-    pair_weight_.resize(n_trees_);
-    pair_weight_.upload(weights.data(), n_trees_, s);
+        meta[padded + 2 * n_trees_ + o] =
+            (uint32_t)(std::lower_bound(outputs.begin(), outputs.end(), o) - outputs.begin());
+    pair_meta_.resize(meta.size());
+    pair_meta_.upload(meta.data(), meta.size(), s);
     dev_.sync();  // the uploads have read this call's arrays
     pair_levels_ = levels;
     pairs_ok_ = true;
@@ -323,7 +324,7 @@ uint32_t Forest::pair_waves(uint64_t blocks, uint64_t block_bytes) const {
     } else if (resident(1) < (n_trees_ >= 256 ? 16 : 6)) {
         for (w = 2; w < 8 && resident(w) <= 12;) w *= 2;
     }
-    w = std::min<uint64_t>(w, (n_trees_ + 15) / 16);
+    w = std::min<uint64_t>(w, (n_trees_ + kPairGroup - 1) / kPairGroup);
     while (w > 1 && resident(w) == 0) w--;
     return (uint32_t)w;
 }
@@ -394,10 +395,11 @@ void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float m
         a.pair_values = pair_values_.get();
         a.pair_orig = pair_orig_.get();
         a.pair_levels = pair_levels_;
-        a.pair_tree = pair_tree_.get();
-        a.pair_output = pair_output_.get();
-        a.pair_weight = pair_weight_.get();
-        a.pair_first = pair_first_.get();
+        const size_t padded = (n_trees_ + kPairGroup - 1) / kPairGroup * kPairGroup;
+        a.pair_weight = reinterpret_cast<const float *>(pair_meta_.get());
+        a.pair_tree = pair_meta_.get() + padded;
+        a.pair_output = a.pair_tree + n_trees_;
+        a.pair_first = a.pair_output + n_trees_;
         predict_pairs(a, mirror_block, nan);
         return;
     }

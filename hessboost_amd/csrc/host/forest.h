@@ -67,8 +67,7 @@ private:
     DBuf<PairRecord> pairs_;
     DBuf<uint32_t> pair_values_;
     DBuf<int32_t> pair_orig_;
-    DBuf<uint32_t> pair_tree_, pair_output_, pair_first_;
-    DBuf<float> pair_weight_;
+    DBuf<uint32_t> pair_meta_;  // weights, trees, outputs and first trees, as predict_device points into it
     void build_pairs(const hbr_forest_desc &fd);
     uint32_t pair_waves(uint64_t blocks, uint64_t block_bytes) const;
     void predict_pairs(PredictArgs a, uint64_t block_bytes, bool nan);

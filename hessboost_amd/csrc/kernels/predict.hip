@@ -654,12 +654,20 @@ __device__ __forceinline__ void predict_pairs(const PredictArgs &a) {
         sum.acc = start_margin(a, r, sum.cur);
         for (uint32_t t0 = 0; t0 < a.n_trees; t0 += CH) {
             uint32_t pos[CH], leaf[CH];
+            float weight[CH];  // one scalar load (the table is padded to whole groups)
+#pragma unroll
+            for (int k = 0; k < CH; k++) weight[k] = uniform_load(a.pair_weight, t0 + (uint32_t)k);
             walk_pairs<CH, LEVELS>(a, lane4, t0, pos, leaf);
+            if (ONE && t0 + CH <= a.n_trees) {
+#pragma unroll
+                for (int k = 0; k < CH; k++) sum.acc = sum.acc + weight[k] * __uint_as_float(leaf[k]);
+                continue;
+            }
 #pragma unroll
             for (int k = 0; k < CH; k++) {
                 const uint32_t t = t0 + (uint32_t)k;
                 if (t < a.n_trees) {
-                    const float contrib = uniform_load(a.pair_weight, t) * __uint_as_float(leaf[k]);
+                    const float contrib = weight[k] * __uint_as_float(leaf[k]);
                     if (ONE) {
                         sum.acc = sum.acc + contrib;
                         continue;
@@ -744,8 +752,8 @@ __device__ __forceinline__ void predict_pairs_shared(const PredictArgs &a) {
 
 template <bool MISSING_NAN, bool ONE, bool SHARED, int LEVELS>
 __device__ __forceinline__ void predict_pairs_walk(const PredictArgs &a) {
-    if constexpr (SHARED) predict_pairs_shared<MISSING_NAN, 16, LEVELS, ONE>(a);
-    else predict_pairs<MISSING_NAN, 16, LEVELS, ONE>(a);
+    if constexpr (SHARED) predict_pairs_shared<MISSING_NAN, kPairGroup, LEVELS, ONE>(a);
+    else predict_pairs<MISSING_NAN, kPairGroup, LEVELS, ONE>(a);
 }
 
 template <bool MISSING_NAN, bool ONE, bool SHARED>
