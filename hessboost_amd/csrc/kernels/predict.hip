@@ -720,14 +720,19 @@ __device__ __forceinline__ void predict_pairs_shared(const PredictArgs &a) {
             const uint32_t t0 = c0 + wave * CH;
             if (t0 < a.n_trees) {
                 uint32_t pos[CH], leaf[CH];
-                walk_pairs<CH, LEVELS>(a, lane4, t0, pos, leaf);
+                float weight[CH];
 #pragma unroll
-                for (int k = 0; k < CH; k++) {
-                    const uint32_t t = t0 + (uint32_t)k;
-                    if (t < a.n_trees) {
-                        s_val[(wave * CH + (uint32_t)k) * kPredPitch + lane] =
-                            uniform_load(a.pair_weight, t) * __uint_as_float(leaf[k]);
-                        if (!ONE && a.leaf_out && lane < rows)
+                for (int k = 0; k < CH; k++) weight[k] = uniform_load(a.pair_weight, t0 + (uint32_t)k);
+                walk_pairs<CH, LEVELS>(a, lane4, t0, pos, leaf);
+                // (the values past the last tree are not added)
+#pragma unroll
+                for (int k = 0; k < CH; k++)
+                    s_val[(wave * CH + (uint32_t)k) * kPredPitch + lane] = weight[k] * __uint_as_float(leaf[k]);
+                if (!ONE && a.leaf_out && lane < rows) {
+#pragma unroll
+                    for (int k = 0; k < CH; k++) {
+                        const uint32_t t = t0 + (uint32_t)k;
+                        if (t < a.n_trees)
                             a.leaf_out[(size_t)r * a.n_trees + uniform_load(a.pair_tree, t)] =
                                 a.pair_orig[(size_t)t * leaves + pos[k]];
                     }
