@@ -464,27 +464,26 @@ void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float m
 // - more: in chunks, each staged by the host's threads and copied while the
 //   walk runs on the one before (Device::host_rows); small enough that the
 //   first chunk's copy is little of the whole (500,000 x 30: 2,356 -> 1,450 us).
-// The buffers stay with the forest up to kKeepBytes.
+// The other buffers stay with the forest up to kKeepBytes.
 void Forest::predict_host(const float *x, uint64_t n, uint64_t n_cols, float missing, float *out,
                           const float *init) {
     if (n == 0) return;
     const uint64_t k = n_outputs_;
     const uint64_t row_bytes = n_cols * sizeof(float), out_bytes = n * k * sizeof(float);
     hipStream_t s = dev_.stream();
-    constexpr uint64_t kDirectBytes = 256ull << 10, kPipeBytes = 1ull << 20, kChunkBytes = 128ull << 20;
+    constexpr uint64_t kDirectRows = Device::kDirectBytes / 2, kPipeBytes = 1ull << 20, kChunkBytes = 128ull << 20;
     constexpr uint64_t kKeepBytes = 64ull << 20;
     const bool pairs = n_trees_ && pairs_ok_ && !std::getenv("HBROCM_PRED_KERNEL") &&
                        (n_cols + 1) * (uint64_t)kPredPitch * sizeof(float) <= 40ull * 1024;
-    if (pairs && row_bytes && n * row_bytes + 2 * out_bytes <= kDirectBytes) {
+    if (pairs && row_bytes && n * row_bytes + 2 * out_bytes <= kDirectRows) {
         // rows, outputs and starting margins, each from a 256-byte boundary
         auto padded = [](uint64_t b) { return (b + 255) / 256 * 256; };
         const uint64_t x_bytes = padded(n * row_bytes), o_bytes = padded(out_bytes);
-        char *host = static_cast<char *>(direct_.reserve(2 * kDirectBytes));
-        void *dev = nullptr;
-        HBR_HIP(hipHostGetDevicePointer(&dev, host, 0));
+        const Device::Direct pinned = dev_.direct();
+        char *host = pinned.host;
         std::memcpy(host, x, n * row_bytes);
         if (init) std::memcpy(host + x_bytes + o_bytes, init, out_bytes);
-        float *d = static_cast<float *>(dev);
+        float *d = reinterpret_cast<float *>(pinned.dev);
         predict_device(d, n, n_cols, missing, d + x_bytes / 4, nullptr, init ? d + (x_bytes + o_bytes) / 4 : nullptr);
         dev_.sync();
         std::memcpy(out, host + x_bytes, out_bytes);

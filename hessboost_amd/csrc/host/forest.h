@@ -46,7 +46,6 @@ private:
     DBuf<uint32_t> chunk_tree_, chunk_node_;
     void plan_chunks(uint32_t cap);
     // predict_host's buffers
-    PinnedBuf direct_;
     DBuf<float> host_x_, host_out_, host_init_;
     DBuf<int32_t> orig_;
     DBuf<float> weight_, base_;

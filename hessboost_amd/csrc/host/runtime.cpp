@@ -74,6 +74,7 @@ Device::~Device() {
         }
         (void)hipStreamDestroy(pipe_copy_);
     }
+    if (direct_) (void)hipHostFree(direct_);
     for (auto &p : pending_) {
         (void)hipEventDestroy(p.start);
         (void)hipEventDestroy(p.stop);
@@ -242,6 +243,16 @@ void Device::host_rows(const float *x, uint64_t n, uint64_t n_cols, uint64_t chu
         pipe_used_set_[b] = true;
     }
     HBR_HIP(hipStreamSynchronize(pipe_copy_));
+}
+
+Device::Direct Device::direct() {
+    Direct d{std::unique_lock<std::mutex>(direct_mu_), nullptr, nullptr};
+    if (!direct_) HBR_HIP(hipHostMalloc(&direct_, kDirectBytes, hipHostMallocDefault));
+    void *dev = nullptr;
+    HBR_HIP(hipHostGetDevicePointer(&dev, direct_, 0));
+    d.host = static_cast<char *>(direct_);
+    d.dev = static_cast<char *>(dev);
+    return d;
 }
 
 static std::mutex g_devices_mu;

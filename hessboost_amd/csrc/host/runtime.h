@@ -74,6 +74,18 @@ public:
     void host_rows(const float *x, uint64_t n, uint64_t n_cols, uint64_t chunk_rows,
                    const std::function<void(const float *, uint64_t, uint64_t)> &fn);
 
+    // kDirectBytes of pinned memory that kernels read and write in place,
+    // for a small request's rows and results: the device's, kept until the
+    // process ends (an object's own cost it 0.2 ms to free), and the
+    // caller's while it holds the lock.
+    static constexpr size_t kDirectBytes = 512ull << 10;
+    struct Direct {
+        std::unique_lock<std::mutex> held;
+        char *host;
+        char *dev;
+    };
+    Direct direct();
+
 private:
     void launch_raw(const char *kernel, dim3 grid, dim3 block, const void *args, uint32_t lds_bytes);
     hipFunction_t function(const char *kernel);
@@ -104,6 +116,8 @@ private:
     float *pipe_rows_[2] = {nullptr, nullptr};
     bool pipe_used_set_[2] = {false, false};
     uint64_t pipe_bytes_ = 0;
+    std::mutex direct_mu_;
+    void *direct_ = nullptr;
 };
 
 // The process's Device for an ordinal (created on first use).
