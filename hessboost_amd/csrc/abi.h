@@ -779,15 +779,13 @@ struct LeafArgs {
     uint32_t n_tiles;
 };
 
-// A grown tree routed over the binned rows: node meta is feature (bits
-// 0-14) | default_left << 15 | limit << 16 | leaf << 31 (present local bins
-// below `limit` go left, a missing value the default way), left child
-// absolute with the right child at left + 1, leaf values as f32.
+// A grown tree routed over the binned rows by its records (present local
+// bins below a node's `limit` go left, a missing value the default way).
+// Walks that hold the tree in LDS (rows of at most 64 features) pack a node
+// into two words: feature (bits 0-14) | default_left << 15 | limit << 16 |
+// leaf << 31, and the left child.
 constexpr uint32_t kMetaDefaultLeft = 1u << 15;
 struct WalkArgs {
-    const uint32_t *meta;
-    const uint32_t *left;
-    const float *value;
     const uint8_t *bins8;        // dense row-major local bins [n][stride]
     float *margins;
     uint32_t stride;
@@ -796,10 +794,8 @@ struct WalkArgs {
     uint32_t output;
     uint32_t n_nodes;
     uint32_t guard_n;            // QScale records the guard checks (0 counts as 1)
-    // A device-grown tree is read from its records (n_nodes from counts)
-    // instead of meta/left/value.
     const GrowTreeNode *tree;
-    const GrowCounts *counts;
+    const GrowCounts *counts;    // non-null (a device-grown tree): n_nodes is read from here
     // Non-null: the walk (and the gradients) happen only when the gradients
     // the tree was grown from were final (no rows left to the host, none
     // non-finite in any of the guard_n scales: a softmax round's classes)
@@ -808,8 +804,7 @@ struct WalkArgs {
     const QScale *guard;
     uint32_t *poison;
     // Rows carry missing masks (their words from byte mask_at): a masked
-    // feature sends the row the way of the node's default (meta bit 15 set:
-    // left).
+    // feature sends the row the way of the node's default.
     uint32_t masked;
     uint32_t mask_at;
     // hbr_walk_leaves_batch: trees walked in one pass over the rows; tree c's

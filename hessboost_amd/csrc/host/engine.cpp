@@ -2355,33 +2355,20 @@ bool Engine::can_walk_gradients(size_t n_nodes) const {
     return dense_u8_ && stride_ == 32 && n_nodes <= 1024 && outputs_ == 1 && labels_loaded_;
 }
 
-void Engine::walk_add(const std::vector<uint32_t> &meta, const std::vector<uint32_t> &left,
-                      const std::vector<float> &value, uint32_t output, const hbr_device_loss *next_loss) {
+void Engine::walk_add(const std::vector<GrowTreeNode> &nodes, uint32_t output, const hbr_device_loss *next_loss) {
     if (!dense_u8_) fail(kRefused, "walk_add: the index has no row-major u8 bins");
-    const size_t n = meta.size();
-    if (n == 0 || left.size() != n || value.size() != n) fail(kInvalid, "walk_add: one meta, left, value per node");
-    for (size_t i = 0; i < n; i++) {
-        if (meta[i] >> 31) continue;
-        if ((meta[i] & (kMetaDefaultLeft - 1u)) >= n_cols_ || (uint64_t)left[i] + 1 >= n)
+    const size_t n = nodes.size();
+    if (n == 0) fail(kInvalid, "walk_add: a tree without nodes");
+    for (const GrowTreeNode &nd : nodes)
+        if (nd.left >= 0 && (nd.feature >= n_cols_ || (uint64_t)nd.left + 1 >= n))
             fail(kInvalid, "walk_add: a split names a missing feature or child");
-    }
     if (output >= outputs_) fail(kInvalid, "walk_add: no such output");
     hipStream_t s = dev_.stream();
-    // the three node tables in one upload
-    const size_t bytes = 3 * n * sizeof(uint32_t);
-    char *host = static_cast<char *>(stage_.alloc(bytes));
-    std::memcpy(host, meta.data(), n * 4);
-    std::memcpy(host + n * 4, left.data(), n * 4);
-    std::memcpy(host + 2 * n * 4, value.data(), n * 4);
-    d_walk_.reserve(bytes);
-    char *dev = reinterpret_cast<char *>(d_walk_.get());
-    HBR_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s));
+    upload_vec(d_walk_, nodes, stage_, s);
     WalkArgs a{};
     a.masked = masked_ ? 1u : 0u;
     a.mask_at = mask_at_;
-    a.meta = reinterpret_cast<const uint32_t *>(dev);
-    a.left = reinterpret_cast<const uint32_t *>(dev + n * 4);
-    a.value = reinterpret_cast<const float *>(dev + 2 * n * 4);
+    a.tree = d_walk_.get();
     a.bins8 = rows8_.get();
     a.margins = margins_.get();
     a.stride = stride_;
@@ -2416,7 +2403,7 @@ void Engine::walk_add(const std::vector<uint32_t> &meta, const std::vector<uint3
         return;
     }
     dev_.launch(staged ? "hbr_walk_leaves32" : "hbr_walk_leaves", dim3(blocks), dim3(256), a);
-    // the staged node tables are released at the next synchronisation
+    // the staged records are released at the next synchronisation
 }
 
 std::vector<QBin> Engine::build_rows(const uint32_t *rows, uint64_t m) {

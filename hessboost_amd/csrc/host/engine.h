@@ -189,13 +189,12 @@ public:
     std::vector<LevelChild> level(const std::vector<LevelSplit> &splits, bool terminal);
     void add_leaves(const std::vector<Segment> &segs, const std::vector<float> &values, uint32_t output);
     // Dense u8 index: margins of output `output` += the leaf each row reaches
-    // through the tree (meta/left/value as WalkArgs lays them out); needs no
-    // row segments, so the depth limit's level can skip its partition.
+    // through the tree; needs no row segments, so the depth limit's level can
+    // skip its partition.
     bool can_walk() const { return dense_u8_ && n_cat_ == 0; }
     // With next_loss, the same pass also computes the next round's gradients
     // of the updated margins (like compute_gradients_async; can_walk_gradients).
-    void walk_add(const std::vector<uint32_t> &meta, const std::vector<uint32_t> &left,
-                  const std::vector<float> &value, uint32_t output, const hbr_device_loss *next_loss = nullptr);
+    void walk_add(const std::vector<GrowTreeNode> &nodes, uint32_t output, const hbr_device_loss *next_loss = nullptr);
     bool can_walk_gradients(size_t n_nodes) const;
     // ---- depthwise growth on the device ----------------------------------------
     // A whole depthwise tree decided level by level on the device from the
@@ -575,7 +574,7 @@ private:
     DBuf<uint32_t> d_hcounts_;
     DBuf<QBin> d_partial_;
     DBuf<uint64_t> d_decisions_;
-    DBuf<uint8_t> d_walk_;  // a tree's meta, left and value tables, one after another
+    DBuf<GrowTreeNode> d_walk_;  // a host-grown tree
     DBuf<ScanNode> d_snodes_;
     DBuf<ScanBest> d_per_feature_, d_best_;
     // categorical features: rank per feature, feature per rank, their

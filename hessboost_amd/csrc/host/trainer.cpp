@@ -618,24 +618,11 @@ void Trainer::grow_and_add(TreeBuilder &b, uint32_t output, const hbr_device_los
     grads_ready_ = false;
     if (e_.n_eval_sets()) e_.walk_evals(records_of(t), output, nullptr, eval_cats_of(t).get());
     if (walk) {
-        const size_t n = t.nodes.size();
-        std::vector<uint32_t> meta(n), left(n, 0);
-        std::vector<float> value(n, 0.0f);
-        for (size_t i = 0; i < n; i++) {
-            const TreeNode &nd = t.nodes[i];
-            if (nd.left < 0) {
-                meta[i] = 1u << 31;
-                value[i] = nd.leaf_value;
-            } else {
-                meta[i] = nd.split_feature | (nd.default_left ? kMetaDefaultLeft : 0u) | (nd.split_limit << 16);
-                left[i] = (uint32_t)nd.left;
-            }
-        }
-        if (next_loss && e_.can_walk_gradients(n)) {
-            e_.walk_add(meta, left, value, output, next_loss);
+        if (next_loss && e_.can_walk_gradients(t.nodes.size())) {
+            e_.walk_add(records_of(t), output, next_loss);
             grads_ready_ = true;
         } else {
-            e_.walk_add(meta, left, value, output);
+            e_.walk_add(records_of(t), output);
         }
         return;
     }
@@ -837,7 +824,7 @@ static std::unique_ptr<Engine::EvalCats> eval_cats_of(const Tree &t) {
 }
 
 // A tree's nodes as the device walks read them: split bin (the threshold is
-// its cut value), feature, default direction, children, leaf value.
+// its cut value) and limit, feature, default direction, children, leaf value.
 std::vector<GrowTreeNode> records_of(const Tree &t) {
     std::vector<GrowTreeNode> r(t.nodes.size());
     for (size_t i = 0; i < t.nodes.size(); i++) {
@@ -849,6 +836,7 @@ std::vector<GrowTreeNode> records_of(const Tree &t) {
         if (n.left < 0) continue;
         g.feature = n.split_feature;
         g.bin = (int32_t)n.split_bin;
+        g.limit = n.split_limit;
         g.default_left = n.default_left;
     }
     return r;

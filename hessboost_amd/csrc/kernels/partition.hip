@@ -399,24 +399,20 @@ extern "C" __global__ __launch_bounds__(256) void hbr_add_leaves(LeafArgs a) {
     }
 }
 
-// The same margins update for a dense u8 index, in row order: each row is
+// The same margins update for a dense index, in row order: each row is
 // routed down the grown tree on its own local bins (the routing of the
 // partition: bin < limit goes left), so the last level needs no partition
 // and the margins are read and written once, coalesced. A node table that
 // does not lead to a leaf within n_nodes steps leaves the row unchanged.
 // The node count of the walked tree: given, or from a device-grown tree's
-// counts (whose records are then read instead of meta/left/value; a leaf's
-// left is -1).
-__device__ __forceinline__ uint32_t walk_nodes(const WalkArgs &a) { return a.tree ? a.counts->n_nodes : a.n_nodes; }
+// counts.
+__device__ __forceinline__ uint32_t walk_nodes(const WalkArgs &a) { return a.counts ? a.counts->n_nodes : a.n_nodes; }
 
-__device__ __forceinline__ uint32_t node_meta(const WalkArgs &a, uint32_t i, uint32_t *left) {
-    if (!a.tree) {
-        *left = a.left[i];
-        return a.meta[i];
-    }
-    const GrowTreeNode t = a.tree[i];
-    *left = t.left < 0 ? 0u : (uint32_t)t.left;
-    return t.left < 0 ? 1u << 31 : t.feature | (t.default_left ? kMetaDefaultLeft : 0u) | (t.limit << 16);
+// A node of the walks that hold the tree in LDS: its packed word and left
+// child (rows of at most 64 features).
+__device__ __forceinline__ uint2 packed_node(const GrowTreeNode &t) {
+    if (t.left < 0) return make_uint2(1u << 31, 0u);
+    return make_uint2(t.feature | (t.default_left ? kMetaDefaultLeft : 0u) | (t.limit << 16), (uint32_t)t.left);
 }
 
 // A guarded walk that must not happen: the tree's gradients (any of its
@@ -431,27 +427,26 @@ __device__ __forceinline__ bool walk_skipped(const WalkArgs &a) {
     return bad != 0;
 }
 
+// Any number of features: the records are read as they are, not packed.
 template <typename Bin>
 __device__ __forceinline__ void walk_leaves(const WalkArgs &a, const Bin *bins) {
     if (walk_skipped(a)) return;
     const uint32_t n_nodes = walk_nodes(a);
     for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < a.n; r += gridDim.x * blockDim.x) {
         const Bin *b = bins + (size_t)r * a.stride;
-        uint32_t nid = 0, left;
-        uint32_t meta = node_meta(a, 0, &left);
-        for (uint32_t step = 0; step < n_nodes && !(meta >> 31); step++) {
-            const uint32_t f = meta & (kMetaDefaultLeft - 1u), lim = (meta >> 16) & 0x7fffu;
-            // masked rows: feature f's bit of its group's mask word
+        GrowTreeNode nd = a.tree[0];
+        for (uint32_t step = 0; step < n_nodes && nd.left >= 0; step++) {
+            // masked rows: the feature's bit of its group's mask word
+            const uint32_t f = nd.feature;
             const uint32_t mask =
                 a.masked ? *reinterpret_cast<const uint32_t *>(b + a.mask_at + 4 * (f >> 5)) >> (f & 31u) : 0u;
-            const bool right = (mask & 1u) ? !(meta & kMetaDefaultLeft) : (uint32_t)b[f] >= lim;
-            nid = left + (right ? 1u : 0u);
-            nid = nid < n_nodes ? nid : 0u;
-            meta = node_meta(a, nid, &left);
+            const bool right = (mask & 1u) ? !nd.default_left : (uint32_t)b[f] >= nd.limit;
+            const uint32_t nid = (uint32_t)nd.left + (right ? 1u : 0u);
+            nd = a.tree[nid < n_nodes ? nid : 0u];
         }
-        if (meta >> 31) {
+        if (nd.left < 0) {
             float *m = a.margins + (size_t)r * a.m_stride + a.output;
-            *m = *m + (a.tree ? a.tree[nid].value : a.value[nid]);
+            *m = *m + nd.value;
         }
     }
 }
@@ -521,9 +516,7 @@ __device__ __forceinline__ void walk_leaves_batch(const WalkArgs &a) {
         const uint32_t first = s_first[c], n = s_first[c + 1] - first;
         for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
             const GrowTreeNode t = tc[i];
-            const uint32_t meta =
-                t.left < 0 ? 1u << 31 : t.feature | (t.default_left ? kMetaDefaultLeft : 0u) | (t.limit << 16);
-            s_node[first + i] = make_uint2(meta, t.left < 0 ? 0u : (uint32_t)t.left);
+            s_node[first + i] = packed_node(t);
             s_value[first + i] = t.value;
         }
     }
@@ -582,20 +575,9 @@ extern "C" __global__ __launch_bounds__(256) void hbr_walk_leaves_batch64(WalkAr
 __device__ __forceinline__ uint32_t load_walk_nodes(const WalkArgs &a, uint2 *s_node, float *s_value) {
     const uint32_t n_nodes = min(walk_nodes(a), kWalkLdsNodes);
     for (uint32_t i = threadIdx.x; i < n_nodes; i += blockDim.x) {
-        uint32_t meta, left;
-        float value;
-        if (a.tree) {
-            const GrowTreeNode t = a.tree[i];
-            meta = t.left < 0 ? 1u << 31 : t.feature | (t.default_left ? kMetaDefaultLeft : 0u) | (t.limit << 16);
-            left = t.left < 0 ? 0u : (uint32_t)t.left;
-            value = t.value;
-        } else {
-            meta = a.meta[i];
-            left = a.left[i];
-            value = a.value[i];
-        }
-        s_node[i] = make_uint2(meta, left);
-        s_value[i] = value;
+        const GrowTreeNode t = a.tree[i];
+        s_node[i] = packed_node(t);
+        s_value[i] = t.value;
     }
     return n_nodes;
 }
