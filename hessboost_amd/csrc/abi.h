@@ -344,7 +344,8 @@ struct HistNode {
     uint32_t contiguous; // rows are seg.offset .. seg.offset+len (no row buffer)
     uint32_t tile_begin; // first row tile (written by the plan kernel)
     uint32_t n_tiles;    // row tiles of the node (written by the plan kernel)
-    uint32_t pad[2];     // [0]: first partial of a multi-tile node (of every node of a device-grown level); [1]: parent slot + 1 of a
+    uint32_t pad[2];     // [0]: first partial of a multi-tile node (PlanArgs::all_partials: of
+                         // every node); [1]: parent slot + 1 of a
                          // split's built child, whose sibling = parent - built as bins complete
                          // (dense kernels; both written by the plan kernel)
     uint32_t cls;        // class (tree) of a batched level: pairs at gpair + cls * class_rows,
@@ -367,9 +368,9 @@ struct PlanArgs {
     uint32_t *counts;           // [0] tiles, [1] tile_rows
     uint32_t min_cost;          // a tile's fixed cost in rows' (Engine::tile_cost)
     uint32_t fuse_subtract;     // built children of splits also update their siblings (dense kernels)
-    // non-null: one node per split of the level, n_splits read from here; every
-    // node's tiles have partials
-    const GrowCounts *grow;
+    const GrowCounts *grow;     // non-null: one node per split of the level, n_splits read from here
+    uint32_t all_partials;      // a node of one tile has a partial too (HistArgs::partials_only)
+    uint32_t pad;
 };
 
 // The reference's CPU histogram in its own f64 order (replays): one

@@ -1292,6 +1292,23 @@ uint32_t Engine::csr_lanes(uint32_t groups, bool ranges) const {
     return lanes;
 }
 
+// Whether a device-grown level of up to n splits leaves its reduce to the
+// search (hbr_reduce_scan), for which every node has a partial beside the
+// `shared` ones of the nodes of several tiles (both in bins): 128 KiB a node
+// and 32 features, and a workgroup of 512 threads a feature, however few its
+// bins. Features that fill them gain at every level (60k x 1,000 rows of ~250
+// bins, ms a tree of depth 5 / 8 / 11: 0.59 / 2.13 / 8.6, in two launches 0.64
+// / 2.22 / 10.3), those of 128 break even (0.59 / 2.10 / 12.0 against 0.64 /
+// 2.02 / 11.6), and fewer lose as soon as the workgroups are many (64: 0.57 /
+// 2.00 / 11.5 against 0.59 / 1.63 / 8.7; 32 features: 0.27 / 0.47 / 0.98
+// against 0.28 / 0.48 / 0.91).
+bool Engine::scan_reduces(uint32_t n, size_t shared, size_t per_node) const {
+    if ((uint64_t)total_bins_ < 160ull * n_cols_ && (uint64_t)n * n_cols_ > 8192) return false;
+    if (d_partial_.size() >= shared + n * per_node) return true;
+    size_t free_b = 0, total_b = 0;
+    return hipMemGetInfo(&free_b, &total_b) == hipSuccess && n * per_node * sizeof(QBin) <= free_b / 4;
+}
+
 // Histograms of a batch of nodes into their slots: the plan kernel cuts the
 // nodes' rows into tiles (about `per_cu` resident workgroups per CU over the
 // launch), then one workgroup per (tile, feature group). Dense u8 tiles
@@ -1308,8 +1325,6 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     const uint32_t fg = wide ? fg16_ : masked_ ? 32u : hist_features_per_group;  // masked rows: fg32 groups
     const uint32_t group_bins = wide ? kWideLdsBins / fg16_ : 256u;
     const bool dense = dense_u8_ || wide;
-    // a device-grown level's partials of u8 rows are summed by its search
-    const bool reduce_in_scan = grow && dense_u8_;
     // dense: feature groups of fg features; CSR: ranges of kCsrGroupBins
     // global bins (every range of every tile is written: no slot zeroing)
     const uint32_t groups = dense ? ceil_div(n_cols_, fg) : ceil_div(total_bins_, kCsrGroupBins);
@@ -1319,7 +1334,10 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     (void)host_nodes;
     d_htiles_.reserve(target + n);
     d_hcounts_.reserve(4);
-    d_partial_.reserve((size_t)(2 * target + (grow ? n : 0u)) * groups * (dense ? fg * group_bins : kCsrGroupBins));
+    const size_t tile_bins = (size_t)groups * (dense ? fg * group_bins : kCsrGroupBins);
+    // a device-grown level's partials of u8 rows are summed by its search
+    reduce_in_scan_ = grow && dense_u8_ && scan_reduces(n, 2 * target * tile_bins, tile_bins);
+    d_partial_.reserve((2 * target + (reduce_in_scan_ ? n : 0u)) * tile_bins);
 
     HistNode *nodes_rw = const_cast<HistNode *>(nodes_dev);  // the plan kernel resolves them in place
     PlanArgs p{};
@@ -1331,8 +1349,9 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     p.tiles = d_htiles_.get();
     p.counts = d_hcounts_.get();
     p.min_cost = tile_cost(groups);
-    p.fuse_subtract = dense && !reduce_in_scan ? 1u : 0u;
+    p.fuse_subtract = dense && !reduce_in_scan_ ? 1u : 0u;
     p.grow = grow;
+    p.all_partials = reduce_in_scan_ ? 1u : 0u;
     dev_.launch("hbr_hist_plan", dim3(1), dim3(256), p);
 
     HistArgs a{};
@@ -1364,7 +1383,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
     a.min_hess = row_pairs_min_hess_;
     a.bins16 = rows16_.get();
     a.stride16 = stride16_;
-    a.partials_only = reduce_in_scan ? 1u : 0u;
+    a.partials_only = reduce_in_scan_ ? 1u : 0u;
     static const char *const wide_kernels[] = {"hbr_hist_dense16_fg1", "hbr_hist_dense16_fg2", "hbr_hist_dense16_fg4",
                                                "hbr_hist_dense16_fg8", "hbr_hist_dense16_fg16"};
     const char *k = wide ? wide_kernels[__builtin_ctz(fg)] : !dense_u8_ ? "hbr_hist_csr" : dense8_kernel(fg);
@@ -1392,7 +1411,7 @@ void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vecto
         r.grow = grow;
         r.group_bins = group_bins;
         r.quarters = group_bins / 64u;
-        if (!reduce_in_scan) dev_.launch("hbr_hist_reduce", dim3(n_cols_ * r.quarters, n), dim3(1024), r);
+        if (!reduce_in_scan_) dev_.launch("hbr_hist_reduce", dim3(n_cols_ * r.quarters, n), dim3(1024), r);
     }
 }
 
@@ -1464,7 +1483,7 @@ void Engine::launch_scan(const ScanNode *nodes_dev, uint32_t n, const PartSplit 
     // a sparse level's search does
     const bool sparse = !dense_u8_ && !dense16_;
     a.subtract = sparse && splits_dev ? 1u : 0u;
-    if (grow && dense_u8_)  // both children of each split; launch_hist left the reduce to it
+    if (grow && reduce_in_scan_)  // both children of each split; launch_hist left the reduce to it
         dev_.launch("hbr_reduce_scan", dim3(n_cols_, n / 2), dim3(512), ReduceScanArgs{reduce_args_, a});
     else
         dev_.launch(sparse ? "hbr_scan_sparse" : "hbr_scan_features", dim3(ceil_div(pairs, 4)), dim3(256), a);
@@ -1706,7 +1725,8 @@ std::vector<LevelChild> Engine::level(const std::vector<LevelSplit> &splits, boo
 // a copy and a wait each way on the host's path and three partition launches
 // (500k x 28 rows of 512 bins, depth 7: 107 us a level, decided here 80).
 bool Engine::can_grow_device(uint64_t max_depth, uint32_t n_trees) const {
-    if (!device_grow || !(dense_u8_ || (dense16_ && cols16_.size())) || max_depth < 1 || max_depth > kMaxDeviceDepth || n_rows_ == 0) return false;
+    if (!device_grow || !(dense_u8_ || (dense16_ && cols16_.size()))) return false;
+    if (max_depth < 1 || max_depth > kMaxDeviceDepth || n_rows_ == 0) return false;
     if (n_cat_) return false;  // categorical splits are decided by the host
     if (n_trees < 1 || n_trees > kGrowMaxTrees || (uint64_t)n_trees * n_rows_ > UINT32_MAX) return false;
     const uint64_t slots = (uint64_t)n_trees << (max_depth - 1);

@@ -377,9 +377,11 @@ private:
                      const GrowCounts *grow = nullptr);
     void launch_scan(const ScanNode *nodes_dev, uint32_t n, const PartSplit *splits_dev, const PartOut *part_out_dev,
                      ScanBest *best_dev, const GrowCounts *grow = nullptr, uint32_t *best_sets_dev = nullptr);
-    // the last launch_hist's reduce: a device-grown level's launch_scan does
-    // it in the same launch
+    // the last launch_hist's reduce, which a device-grown level's launch_scan
+    // does in the same launch when reduce_in_scan_ is set
     ReduceArgs reduce_args_{};
+    bool reduce_in_scan_ = false;
+    bool scan_reduces(uint32_t n, size_t shared, size_t per_node) const;
     // the root's total, histogram and split search, queued (no synchronisation)
     void launch_root(const Segment &seg, uint32_t slot, float lower, float upper);
     // the roots of a device-grown batch (root t in slot t, of class t,

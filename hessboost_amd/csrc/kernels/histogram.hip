@@ -369,7 +369,7 @@ extern "C" __global__ __launch_bounds__(256) void hbr_hist_plan(PlanArgs a) {
         const uint32_t n = (len + tile_rows - 1) / tile_rows;
         uint32_t all, part_all;
         const uint32_t first = block_exclusive_scan<256>(n, &all);
-        const uint32_t part_first = block_exclusive_scan<256>(n > 1 || a.grow ? n : 0u, &part_all);
+        const uint32_t part_first = block_exclusive_scan<256>(n > 1 || a.all_partials ? n : 0u, &part_all);
         if (i < n_nodes) {
             a.nodes[i].tile_begin = carry + first;
             a.nodes[i].n_tiles = n;

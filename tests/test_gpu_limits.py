@@ -1,5 +1,7 @@
 """Calls at the limits of a dispatch: more features than a packed node holds,
 small and uneven shapes that a rule made for average ones must still take."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -47,3 +49,43 @@ def test_trees_over_more_than_32768_features_walk_their_own_features(monkeypatch
     trees = t.trees()
     assert max(int(k["split_feature"].max()) for k in trees) >= 32_768
     assert np.array_equal(t.margins(), _walked(trees, x, t.base_score()[0]))
+
+
+def _free_bytes():
+    """The device's free memory, from the HIP runtime the library has loaded."""
+    hip = C.CDLL("libamdhip64.so.7")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _fit(monkeypatch, x, y, params, device):
+    monkeypatch.setenv("HBROCM_DEVICE_GROW", "1" if device else "0")
+    engine = hb.DMatrix(x, label=y).engine(params["max_bin"])
+    t = hb.Trainer(engine, params, y)
+    free = _free_bytes()
+    t.boost(2)
+    return t.trees(), t.margins(), free - _free_bytes()
+
+
+# few bins a feature beside one of many (a tile's sums take 128 KiB for every
+# feature then), and many features of two bins (128 KiB for every 32): a deep
+# level's nodes may not each take that much
+@pytest.mark.parametrize("f,depth,widest,max_bin", [(300, 10, 5_000, 5_000), (2_000, 11, 2, 256), (2_000, 12, 2, 256),
+                                                    (33, 10, 2, 256)])
+def test_deep_levels_of_few_bins_take_little_memory(monkeypatch, f, depth, widest, max_bin):
+    rng = np.random.default_rng(f + depth)
+    n = 6_000
+    x = rng.integers(0, 2, (n, f)).astype(np.float32)
+    if widest > 2:
+        x[:, 5] = rng.permutation(n).astype(np.float32)
+    y = (x[:, :12] @ rng.standard_normal(12) + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    params = {"objective": "reg:squarederror", "max_depth": depth, "eta": 0.3, "max_bin": max_bin}
+    trees, margins, used = _fit(monkeypatch, x, y, params, True)
+    want, want_margins, _ = _fit(monkeypatch, x, y, params, False)
+    for a, b in zip(trees, want):
+        for key in a:
+            assert np.array_equal(a[key], b[key]), key
+    assert np.array_equal(margins, want_margins)
+    # slots, records and the tiles' partials; a partial a node would take 4 to 10 GB
+    assert used <= 1 << 30, used
