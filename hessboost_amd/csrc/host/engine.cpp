@@ -78,6 +78,7 @@ void Engine::read_tunables() {
     if (const char *v = std::getenv("HBROCM_BATCH_WALK")) batch_walk = std::strtol(v, nullptr, 10) != 0;
     if (const char *v = std::getenv("HBROCM_BIN_ROWS_IN_REGISTERS")) bin_rows_in_registers = std::strtol(v, nullptr, 10) != 0;
     if (const char *v = std::getenv("HBROCM_DEVICE_GROW")) device_grow = std::strtol(v, nullptr, 10) != 0;
+    if (const char *v = std::getenv("HBROCM_HIST_SLOTS")) most_slots = std::strtoull(v, nullptr, 10);
     if (const char *v = std::getenv("HBROCM_CSR_RANGES")) csr_range_table = std::strtol(v, nullptr, 10) != 0;
     if (const char *v = std::getenv("HBROCM_WALK_BLOCKS")) {
         const long b = std::strtol(v, nullptr, 10);
@@ -1219,6 +1220,7 @@ void Engine::free_slot(uint32_t s) { free_slots_.push_back(s); }
 
 bool Engine::reserve_slots(uint64_t n) {
     if (n <= slot_cap_) return true;
+    if (n > most_slots) return false;
     size_t free_b = 0, total_b = 0;
     HBR_HIP(hipMemGetInfo(&free_b, &total_b));
     const uint64_t bytes = n * (uint64_t)total_bins_ * sizeof(QBin);
@@ -1738,7 +1740,7 @@ bool Engine::can_grow_device(uint64_t max_depth, uint32_t n_trees) const {
     if (2 * pmax * n_cols_ > (uint64_t(1) << 22)) return false;
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
-    return std::max<uint64_t>(slots, slot_cap_) * (uint64_t)total_bins_ * sizeof(QBin) <= free_b / 2;
+    return slots <= slot_cap_ || slots * (uint64_t)total_bins_ * sizeof(QBin) <= free_b / 2;
 }
 
 // The roots of a device-grown batch of n_trees trees: their histogram and

@@ -606,6 +606,7 @@ public:
     bool batch_walk = true;  // a softmax round's class trees added to the margins in one walk
     bool bin_rows_in_registers = true;  // device binning of <= 32 features: rows into registers, else staged in LDS
     bool device_grow = true;     // depthwise trees decided on the device where eligible
+    uint64_t most_slots = UINT32_MAX;  // histogram slots the pool may hold
     bool csr_range_table = true; // CSR histograms read each bin range's entries from a per-row table
     uint32_t walk_blocks_per_cu = 4;  // workgroups per CU of the device-tree margin walk (one resident wave)
 };

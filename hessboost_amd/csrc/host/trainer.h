@@ -102,7 +102,10 @@ private:
     LevelSplit split_of(const Open &o, const Decision &d, double cb[4]) const;
     std::vector<uint32_t> set_codes(const Decision &d) const;
     void record(Tree &t, const Open &o, const Decision &d, const double cb[4]);
-    void split_ahead(Open &o, std::vector<Open> &heap, uint64_t leaves_left, uint64_t limit);
+    bool split_ahead(Open &o, std::vector<Open> &heap, uint64_t leaves_left, uint64_t limit);
+    // grow(), best-first trees with splits ahead or without; *redo: the
+    // splits ahead left too few histogram slots, nothing came of the tree
+    Tree grow_tree(std::vector<std::pair<Segment, float>> *leaves, bool walk, bool ahead, bool *redo);
     // Expand node o by d: children appended to the tree; returns the level split.
     LevelSplit expand(Tree &t, const Open &o, const Decision &d, double cb[4]);
     void leaf(const Open &o);
@@ -115,7 +118,10 @@ private:
     std::vector<double> g_, h_, lower_, upper_;
     std::vector<std::pair<int32_t, Segment>> leaves_;
     std::deque<Ahead> ahead_;
-    bool speculate_ = false;
+    uint64_t ahead_most_ = 0;    // most leaves the tree can have, and most splits ahead unused; 0: none ahead
+    uint64_t ahead_unused_ = 0;  // splits ahead whose node has not been popped
+    bool ahead_fits_ = true;     // no tree yet was grown again for want of slots
+    uint64_t ahead_hits_ = 0;    // and those whose node has
 };
 
 struct TrainParams {

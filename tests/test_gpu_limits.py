@@ -89,3 +89,50 @@ def test_deep_levels_of_few_bins_take_little_memory(monkeypatch, f, depth, wides
     assert np.array_equal(margins, want_margins)
     # slots, records and the tiles' partials; a partial a node would take 4 to 10 GB
     assert used <= 1 << 30, used
+
+
+def _best_first(x, y, leaves, depth, rounds=2, max_bin=256):
+    engine = hb.DMatrix(x, label=y).engine(max_bin)
+    params = {"grow_policy": "lossguide", "max_depth": depth, "max_leaves": leaves, "eta": 0.3, "min_child_weight": 2.0}
+    t = hb.Trainer(engine, params, y)
+    free = _free_bytes()
+    before = engine.counters()
+    t.boost(rounds)
+    after = engine.counters()
+    return t, free - _free_bytes(), {k: after[k] - before[k] for k in after}
+
+
+# 1,000 features of 256 bins: 4 MB a histogram slot. A depth limit of 4 leaves
+# no more than 16; where the pops cannot be foreseen the unused splits stay
+# within the leaves, and most pops then split nothing ahead
+@pytest.mark.parametrize("leaves,depth,slots", [(0, 4, 2 * 16), (100, 0, 2 * 100), (3, 0, 2 * 3)])
+def test_best_first_slots_stay_within_twice_the_leaves(leaves, depth, slots):
+    rng = np.random.default_rng(leaves)
+    x = rng.standard_normal((3_000, 1_000), dtype=np.float32)
+    y = rng.standard_normal(3_000).astype(np.float32)
+    t, used, counters = _best_first(x, y, leaves, depth)
+    # 272 partials of 128 KiB a tile and 32 features, of 2 x 256 workgroups at most, and small records
+    assert used <= slots * 1_000 * 256 * 16 + (160 << 20), used / 2**20
+    taken = sum(int(np.sum(k["left"] >= 0)) for k in t.trees())
+    # splits made: a root histogram a tree, then one for each split
+    assert counters["hist_nodes"] - 2 <= 2 * taken
+
+
+# a pool that holds a tree's leaves but not the splits ahead beside them: the
+# same trees, none refused, and the counters of what the kept growth did
+@pytest.mark.parametrize("noise", [0.1, 3.0])
+@pytest.mark.parametrize("leaves,pool", [(60, 64), (127, 128), (32, 32)])
+def test_a_full_slot_pool_grows_the_oracles_best_first_trees(monkeypatch, noise, leaves, pool):
+    from oracle import oracle as O
+    from tests.test_gpu_train import compare_trees
+
+    monkeypatch.setenv("HBROCM_HIST_SLOTS", str(pool))
+    rng = np.random.default_rng(leaves)
+    x = rng.standard_normal((2_500, 20), dtype=np.float32)
+    y = (x[:, 0] - x[:, 1] * x[:, 2] + noise * rng.standard_normal(2_500)).astype(np.float32)
+    ref = O.Model(O.Dataset(x), y, O.params(grow_policy=O.GROW_LOSSGUIDE, max_depth=0, max_leaves=leaves,
+                                            min_child_weight=2.0), 3)
+    t, _, counters = _best_first(x, y, leaves, 0, rounds=3)
+    compare_trees(t.trees(), ref.trees())
+    assert np.max(np.abs(t.margins() - ref.margins().reshape(-1))) <= 1e-5
+    assert counters["trees"] == 3
