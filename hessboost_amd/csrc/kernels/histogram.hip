@@ -203,10 +203,18 @@ __device__ __forceinline__ void hist_dense8(const HistArgs &a) {
 // over 31 ranges: 3), so a wave of one row at a time left 60 lanes idle
 // and waited for its chain of loads (id, pointer, range, entries) alone: the
 // root of 100k x 1,000 sparse rows took 1,119 us, with 4 lanes a row 119.
+// The lanes follow the average row, so rows of many more entries than it
+// (more than kCsrSteps steps of its own lanes), when a wave has few of them,
+// go to all its lanes, kCsrWide loads a lane in flight, instead of holding the
+// wave: roots of 100k rows of 5 entries with one of 16,000 among them 257 ->
+// 36 us, with 200 of 1,000 69 -> 26, of Pareto lengths 130 -> 56, of even rows
+// 135 -> 134.
 // Then the range goes to the node's slot (a node of one tile) or to the
 // tile's partial, summed by hbr_hist_reduce_csr. Every range of every tile
 // is written, so slots need no zeroing.
 constexpr uint32_t kCsrRows = 4;
+constexpr uint32_t kCsrSteps = 8;
+constexpr uint32_t kCsrWide = 4;
 
 __device__ __forceinline__ void hist_csr(const HistArgs &a) {
     __shared__ unsigned long long s_g[kCsrGroupBins], s_h[kCsrGroupBins];
@@ -249,6 +257,41 @@ __device__ __forceinline__ void hist_csr(const HistArgs &a) {
         }
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) iters = max(iters, (uint32_t)__shfl_xor((int)iters, d, kWave));
+        if (iters > kCsrSteps) {  // uniform
+            uint64_t wide[kCsrRows];
+            uint32_t n_wide = 0;
+#pragma unroll
+            for (uint32_t u = 0; u < kCsrRows; u++) {
+                wide[u] = __ballot(sub == 0 && e[u] - b[u] > (uint64_t)kCsrSteps * a.csr_lanes);
+                n_wide += (uint32_t)__popcll(wide[u]);
+            }
+            // a wide row costs the wave a step or two
+            if (iters > kCsrSteps + 2 * n_wide) {
+#pragma unroll
+                for (uint32_t u = 0; u < kCsrRows; u++) {
+                    for (uint64_t m = wide[u]; m; m &= m - 1) {
+                        const int src = __ffsll((unsigned long long)m) - 1;
+                        const uint64_t x1 = __shfl((unsigned long long)e[u], src, kWave);
+                        const unsigned long long wg = __shfl(qg[u], src, kWave), wh = __shfl(qh[u], src, kWave);
+                        for (uint64_t x = __shfl((unsigned long long)b[u], src, kWave) + lane_id(); x < x1;
+                             x += kCsrWide * kWave) {
+                            uint32_t d[kCsrWide];
+#pragma unroll
+                            for (uint32_t k = 0; k < kCsrWide; k++)
+                                d[k] = x + k * kWave < x1 ? a.gbins[x + k * kWave] - lo_bin : 0xffffffffu;
+#pragma unroll
+                            for (uint32_t k = 0; k < kCsrWide; k++)
+                                if (d[k] < nb) {
+                                    atomicAdd(&s_g[d[k]], wg);
+                                    atomicAdd(&s_h[d[k]], wh);
+                                }
+                        }
+                    }
+                    if (e[u] - b[u] > (uint64_t)kCsrSteps * a.csr_lanes) e[u] = b[u];
+                }
+                iters = kCsrSteps;
+            }
+        }
         for (uint32_t k = 0; k < iters; k++) {
             uint32_t d[kCsrRows];
 #pragma unroll

@@ -136,3 +136,31 @@ def test_a_full_slot_pool_grows_the_oracles_best_first_trees(monkeypatch, noise,
     compare_trees(t.trees(), ref.trees())
     assert np.max(np.abs(t.margins() - ref.margins().reshape(-1))) <= 1e-5
     assert counters["trees"] == 3
+
+
+# rows of a few entries among which some are long: a wave of rows with none,
+# with one, with as many long ones as short, ends of waves and of entries
+@pytest.mark.parametrize("f,values", [(300, 3), (4_000, 2), (5_000, 9)])
+@pytest.mark.parametrize("share", [0.0, 0.0005, 0.05, 0.6])
+def test_uneven_sparse_rows_sum_every_entry(f, values, share):
+    rng = np.random.default_rng(f + int(share * 1e4))
+    n = 3_001
+    lens = rng.integers(0, 6, n)
+    lens[rng.random(n) < share] = f - rng.integers(0, 3)
+    lens[-1] = f
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    cols = np.concatenate([np.sort(rng.choice(f, k, replace=False)) for k in lens]).astype(np.int32)
+    vals = rng.integers(0, values, ptr[-1]).astype(np.float32)
+    data = hb.DMatrix((ptr, cols, vals), n_cols=f)
+    engine = data.engine()
+    pairs = rng.integers(-8, 9, (n, 2)).astype(np.float32)  # every sum exact
+    engine.prepare(pairs)
+    row_ptr, row_bins = data.index().row_bins()
+    counts = np.diff(row_ptr.astype(np.int64))
+    for rows in (np.arange(n), np.flatnonzero(rng.random(n) < 0.3), np.array([n - 1]), np.arange(n - 65, n)):
+        hist = engine.build(rows)
+        inside = np.isin(np.repeat(np.arange(n), counts), rows)
+        for c in (0, 1):
+            want = np.bincount(row_bins[inside], weights=np.repeat(pairs[:, c], counts)[inside].astype(np.float64),
+                               minlength=len(hist))
+            assert np.array_equal(hist[:, c], want)
