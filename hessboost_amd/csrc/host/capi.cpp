@@ -60,8 +60,9 @@ int guard(F &&fn) {
 }
 
 // Run fn under the engine's lock; a device error poisons the engine. Rows
-// a trainer reordered go back to the caller's order first, except for the
-// trainer's own calls and those that touch no row (keep_order).
+// a trainer reordered go back to the caller's order first, and the buffers of
+// the reorder with them, except for the trainer's own calls and those that
+// touch no row (keep_order).
 template <typename F>
 int with_engine(hbr_engine *h, F &&fn, bool keep_order = false) {
     if (!h || !h->e) return set_error(HBR_INVALID, "null engine");
@@ -849,6 +850,7 @@ int hbr_kernel_stats(hbr_engine *h, char *buf, size_t len) {
 int hbr_trainer_create(hbr_engine *h, const hbr_train_params *p, const float *labels, const float *weights,
                        uint64_t n, hbr_trainer **out) {
     return with_engine(h, [&](Engine &e) {
+        e.restore_row_order(true);  // the new trainer may reorder the rows again
         if (!p || !labels || !out) fail(kInvalid, "trainer: null argument");
         TrainParams tp;
         tp.grow.reg = reg_from(p->lambda, p->alpha, p->max_delta_step, p->min_child_weight);
@@ -872,7 +874,7 @@ int hbr_trainer_create(hbr_engine *h, const hbr_train_params *p, const float *la
             throw;
         }
         *out = t;
-    });
+    }, true);
 }
 
 int hbr_trainer_boost(hbr_trainer *t, uint64_t rounds) {

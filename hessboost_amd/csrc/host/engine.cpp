@@ -677,13 +677,33 @@ void Engine::order_rows_by_tree() {
     counters.row_orders++;
 }
 
-// The buffers stay with the engine for the next trainer's reorder (freeing
-// them took longer than the gathers).
-void Engine::restore_row_order() {
-    if (!permuted_) return;
-    gather_rows(perm_inv_.get());
-    dev_.sync();
-    permuted_ = false;
+void Engine::restore_row_order(bool keep_buffers) {
+    if (permuted_) {
+        gather_rows(perm_inv_.get());
+        dev_.sync();
+        permuted_ = false;
+    }
+    size_t free_b = 0, total_b = 0;
+    const uint64_t bytes = row_buffer_bytes();
+    if (bytes && !(keep_buffers && hipMemGetInfo(&free_b, &total_b) == hipSuccess && bytes <= free_b / 4))
+        release_row_buffers();
+}
+
+uint64_t Engine::row_buffer_bytes() const {
+    if (permuted_) return 0;
+    const Spare &s = spare_;
+    return s.rows.size() + s.cols.size() + s.pairs.size() * sizeof(GPair) +
+           sizeof(float) * (s.margins.size() + s.labels.size() + s.weights.size() + s.leaf.size() + s.order.size() +
+                            perm_.size() + perm_inv_.size() + group_stamp_.size() + bad_groups_.size());
+}
+
+void Engine::release_row_buffers() {
+    if (permuted_) return;
+    perm_.release();
+    perm_inv_.release();
+    group_stamp_.release();
+    bad_groups_.release();
+    spare_ = Spare{};
 }
 
 void Engine::read_gradients(float *out, uint64_t n) {
@@ -1223,8 +1243,9 @@ bool Engine::reserve_slots(uint64_t n) {
     if (n > most_slots) return false;
     size_t free_b = 0, total_b = 0;
     HBR_HIP(hipMemGetInfo(&free_b, &total_b));
-    const uint64_t bytes = n * (uint64_t)total_bins_ * sizeof(QBin);
-    if (bytes > free_b / 2) return false;
+    const uint64_t bytes = n * (uint64_t)total_bins_ * sizeof(QBin), kept = row_buffer_bytes();
+    if (bytes > (free_b + kept) / 2) return false;
+    if (bytes > free_b / 2) release_row_buffers();
     DBuf<QBin> grown(n * (uint64_t)total_bins_ + 1);
     if (slot_cap_)
         HBR_HIP(hipMemcpyAsync(grown.get(), hist_.get(), (uint64_t)slot_cap_ * total_bins_ * sizeof(QBin),
@@ -1740,7 +1761,7 @@ bool Engine::can_grow_device(uint64_t max_depth, uint32_t n_trees) const {
     if (2 * pmax * n_cols_ > (uint64_t(1) << 22)) return false;
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
-    return slots <= slot_cap_ || slots * (uint64_t)total_bins_ * sizeof(QBin) <= free_b / 2;
+    return slots <= slot_cap_ || slots * (uint64_t)total_bins_ * sizeof(QBin) <= (free_b + row_buffer_bytes()) / 2;
 }
 
 // The roots of a device-grown batch of n_trees trees: their histogram and

@@ -799,6 +799,13 @@ void Trainer::boost(uint64_t rounds) {
     // their candidates and count the nodes they cannot certify
     e_.guard_active = e_.guard_on();
     e_.guard_gamma = (float)p_.grow.gamma;
+    const bool fused = p_.objective != HBR_OBJ_SOFTMAX && p_.grow.policy == HBR_GROW_DEPTHWISE &&
+                       e_.can_walk_device_tree(p_.grow.max_depth);
+    if (fused) {
+        boost_pipelined(rounds, device_loss(), true);
+        return;
+    }
+    e_.release_row_buffers();  // only those rounds reorder the rows
     if (p_.objective == HBR_OBJ_SOFTMAX && p_.grow.policy == HBR_GROW_DEPTHWISE && softmax_batches &&
         e_.can_grow_device(p_.grow.max_depth, k_)) {
         boost_softmax_batched(rounds);
@@ -807,11 +814,6 @@ void Trainer::boost(uint64_t rounds) {
     if (p_.objective == HBR_OBJ_SOFTMAX && p_.grow.policy == HBR_GROW_DEPTHWISE &&
         e_.can_route_device_tree(p_.grow.max_depth)) {
         boost_softmax_pipelined(rounds);
-        return;
-    }
-    if (p_.objective != HBR_OBJ_SOFTMAX && p_.grow.policy == HBR_GROW_DEPTHWISE &&
-        e_.can_walk_device_tree(p_.grow.max_depth)) {
-        boost_pipelined(rounds, device_loss(), true);
         return;
     }
     // wider or masked rows, deeper trees: the same rounds with the walk and

@@ -164,3 +164,37 @@ def test_uneven_sparse_rows_sum_every_entry(f, values, share):
             want = np.bincount(row_bins[inside], weights=np.repeat(pairs[:, c], counts)[inside].astype(np.float64),
                                minlength=len(hist))
             assert np.array_equal(hist[:, c], want)
+
+
+def test_the_reorders_second_copy_of_the_rows_is_given_back(monkeypatch):
+    """After a reordered fit the copy stays for the next such trainer, and
+    goes with the first call of another kind."""
+    monkeypatch.setenv("HBROCM_ROW_ORDER_MIN_ROWS", "1000")
+    rng = np.random.default_rng(4)
+    n = 1_000_000
+    x = rng.standard_normal((n, 20), dtype=np.float32)
+    y = (x[:, 0] + x[:, 1] * x[:, 2] > 0).astype(np.float32)
+    engine = hb.DMatrix(x, label=y).engine()
+    params = {"objective": "binary:logistic", "max_depth": 4}
+    copies = n * (32 + 20 + 4 * 2)  # the rows, the columns, and each row's two places, at least
+
+    def fit(**more):
+        t = hb.Trainer(engine, dict(params, **more), y)
+        t.boost(3)
+        return t.trees(), t.margins()
+
+    first = fit()
+    assert engine.counters()["row_orders"] == 1
+    free = _free_bytes()
+    again = fit()
+    assert abs(_free_bytes() - free) < copies // 4
+    for call in (lambda: engine.load_margins(np.zeros(n, np.float32), 1),
+                 lambda: fit(grow_policy="lossguide", max_leaves=7, max_depth=0)):
+        last = fit()
+        free = _free_bytes()
+        call()
+        assert _free_bytes() - free > copies, (_free_bytes() - free) / 2**20
+    for a, b in zip(first[0] + first[0], again[0] + last[0]):
+        for key in a:
+            assert np.array_equal(a[key], b[key])
+    assert np.array_equal(first[1], last[1]) and np.array_equal(first[1], again[1])
