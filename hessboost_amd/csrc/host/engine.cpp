@@ -841,7 +841,7 @@ GradArgs Engine::grad_args(const hbr_device_loss &loss) {
 
 void Engine::launch_gradients(const hbr_device_loss &loss, uint32_t output) {
     if (!labels_loaded_) fail(kInvalid, "gradients: no labels since load_margins");
-    restore_row_order();  // the gradient kernel's 8-row vectors are consecutive rows
+    restore_row_order(true);  // the gradient kernel's 8-row vectors are consecutive rows
     if (outputs_ != 1 || output != 0) fail(kRefused, "device gradients run for one output");
     hipStream_t s = dev_.stream();
     grains_known_ = false;
@@ -915,7 +915,7 @@ void Engine::softmax_gradients_async(float min_hess) {
     const uint32_t k = outputs_;
     if (k < 1 || k > kSoftmaxMaxClasses) fail(kRefused, "softmax gradients: 1 to 1024 classes");
     if (n_rows_ == 0) fail(kInvalid, "softmax gradients: no rows");
-    restore_row_order();  // the vector batches are consecutive rows
+    restore_row_order(true);  // the vector batches are consecutive rows
     hipStream_t s = dev_.stream();
     row_pairs_live_ = false;
     root_partials_ = 0;  // the staged pairs are no longer the walk's
