@@ -10,6 +10,12 @@
 
 namespace hbr {
 
+struct Forest::PairHost {
+    std::vector<PairRecord> recs;
+    std::vector<uint32_t> values;  // leaf values, then the trees' table
+    std::vector<int32_t> orig;
+};
+
 // Each tree is re-laid out breadth-first so every internal node's children
 // sit side by side (right = left + 1), the node records its original id for
 // leaf queries, and the walk can never loop: every node is reached exactly
@@ -120,7 +126,8 @@ Forest::Forest(int ordinal, const hbr_forest_desc &fd) : dev_(device(ordinal)) {
     up(weight_, weight);
     up(base_, base);
     build_mirror(fd);
-    build_pairs(fd);
+    PairHost held;  // until the copies have read it
+    build_pairs(fd, held);
     dev_.sync();
 }
 
@@ -139,7 +146,7 @@ static float next_below(float c) {
 // The pair layout (PredictArgs::pairs): every tree embedded in the
 // complete tree of the forest's largest depth rounded up to even, a split's
 // first child being the one its missing values take.
-void Forest::build_pairs(const hbr_forest_desc &fd) {
+void Forest::build_pairs(const hbr_forest_desc &fd, PairHost &held) {
     if (has_categorical_ || n_trees_ == 0 || max_feature_ >= 126) return;
     uint32_t depth = 0;
     // depths, and the checks the walk needs
@@ -168,9 +175,14 @@ void Forest::build_pairs(const hbr_forest_desc &fd) {
     uint64_t real = 0;
     for (uint64_t t = 0; t < n_trees_; t++) real += tree_nodes_[t];
     if (bytes > (1ull << 30) || bytes > 64 * real * sizeof(MirrorNode)) return;
-    std::vector<PairRecord> recs(n_trees_ * per_tree);
-    std::vector<uint32_t> values(n_trees_ * leaves);
-    std::vector<int32_t> orig(n_trees_ * leaves);
+    auto &[recs, values, orig] = held;
+    // beside the values, the trees' weights (padded to whole groups of the
+    // walk's trees), numbers and outputs, and each output's first tree: an
+    // allocation and an upload less of a small forest
+    const size_t padded = (n_trees_ + kPairGroup - 1) / kPairGroup * kPairGroup;
+    recs.resize(n_trees_ * per_tree);
+    values.resize(n_trees_ * leaves + padded + 2 * n_trees_ + n_outputs_ + 1);
+    orig.resize(n_trees_ * leaves);
     std::vector<uint32_t> t_at, s_at;  // per complete position of levels < depth
     std::vector<uint32_t> order(n_trees_), outputs(n_trees_);
     std::vector<float> weights(n_trees_);
@@ -227,23 +239,18 @@ void Forest::build_pairs(const hbr_forest_desc &fd) {
     hipStream_t s = dev_.stream();
     pairs_.resize(recs.size() ? recs.size() : 1);
     if (!recs.empty()) pairs_.upload(recs.data(), recs.size(), s);
+    pair_meta_ = n_trees_ * leaves;
+    const auto meta = values.begin() + pair_meta_;
+    std::memcpy(&*meta, weights.data(), n_trees_ * sizeof(float));
+    std::copy(order.begin(), order.end(), meta + padded);
+    std::copy(outputs.begin(), outputs.end(), meta + padded + n_trees_);
+    for (uint32_t o = 0; o <= n_outputs_; o++)
+        meta[padded + 2 * n_trees_ + o] =
+            (uint32_t)(std::lower_bound(outputs.begin(), outputs.end(), o) - outputs.begin());
     pair_values_.resize(values.size());
     pair_values_.upload(values.data(), values.size(), s);
     pair_orig_.resize(orig.size());
     pair_orig_.upload(orig.data(), orig.size(), s);
-    // the trees' weights (padded to whole groups of the walk's trees),
-    // numbers and outputs, and each output's first tree: one upload
-    const size_t padded = (n_trees_ + kPairGroup - 1) / kPairGroup * kPairGroup;
-    std::vector<uint32_t> meta(padded + 2 * n_trees_ + n_outputs_ + 1, 0u);
-    std::memcpy(meta.data(), weights.data(), n_trees_ * sizeof(float));
-    std::copy(order.begin(), order.end(), meta.begin() + padded);
-    std::copy(outputs.begin(), outputs.end(), meta.begin() + padded + n_trees_);
-    for (uint32_t o = 0; o <= n_outputs_; o++)
-        meta[padded + 2 * n_trees_ + o] =
-            (uint32_t)(std::lower_bound(outputs.begin(), outputs.end(), o) - outputs.begin());
-    pair_meta_.resize(meta.size());
-    pair_meta_.upload(meta.data(), meta.size(), s);
-    dev_.sync();  // the uploads have read this call's arrays
     pair_levels_ = levels;
     pairs_ok_ = true;
 }
@@ -396,8 +403,8 @@ void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float m
         a.pair_orig = pair_orig_.get();
         a.pair_levels = pair_levels_;
         const size_t padded = (n_trees_ + kPairGroup - 1) / kPairGroup * kPairGroup;
-        a.pair_weight = reinterpret_cast<const float *>(pair_meta_.get());
-        a.pair_tree = pair_meta_.get() + padded;
+        a.pair_weight = reinterpret_cast<const float *>(pair_values_.get() + pair_meta_);
+        a.pair_tree = pair_values_.get() + pair_meta_ + padded;
         a.pair_output = a.pair_tree + n_trees_;
         a.pair_first = a.pair_output + n_trees_;
         predict_pairs(a, mirror_block, nan);

@@ -66,8 +66,9 @@ private:
     DBuf<PairRecord> pairs_;
     DBuf<uint32_t> pair_values_;
     DBuf<int32_t> pair_orig_;
-    DBuf<uint32_t> pair_meta_;  // weights, trees, outputs and first trees, as predict_device points into it
-    void build_pairs(const hbr_forest_desc &fd);
+    size_t pair_meta_ = 0;  // where in pair_values_ the trees' table starts, as predict_device points into it
+    struct PairHost;
+    void build_pairs(const hbr_forest_desc &fd, PairHost &held);
     uint32_t pair_waves(uint64_t blocks, uint64_t block_bytes) const;
     void predict_pairs(PredictArgs a, uint64_t block_bytes, bool nan);
 };
