@@ -470,7 +470,9 @@ void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float m
 // - up to 1 MiB, or another walk: one copy each way;
 // - more: in chunks, each staged by the host's threads and copied while the
 //   walk runs on the one before (Device::host_rows); small enough that the
-//   first chunk's copy is little of the whole (500,000 x 30: 2,356 -> 1,450 us).
+//   first chunk's copy is little of the whole (500,000 x 30: 2,356 -> 1,450 us)
+//   and the device's staging, which stays, little memory (1.6 GB: 31.6 ms in
+//   chunks of 16 MiB, 34.3 in chunks of 128).
 // The other buffers stay with the forest up to kKeepBytes.
 void Forest::predict_host(const float *x, uint64_t n, uint64_t n_cols, float missing, float *out,
                           const float *init) {
@@ -478,7 +480,7 @@ void Forest::predict_host(const float *x, uint64_t n, uint64_t n_cols, float mis
     const uint64_t k = n_outputs_;
     const uint64_t row_bytes = n_cols * sizeof(float), out_bytes = n * k * sizeof(float);
     hipStream_t s = dev_.stream();
-    constexpr uint64_t kDirectRows = Device::kDirectBytes / 2, kPipeBytes = 1ull << 20, kChunkBytes = 128ull << 20;
+    constexpr uint64_t kDirectRows = Device::kDirectBytes / 2, kPipeBytes = 1ull << 20, kChunkBytes = 16ull << 20;
     constexpr uint64_t kKeepBytes = 64ull << 20;
     const bool pairs = n_trees_ && pairs_ok_ && !std::getenv("HBROCM_PRED_KERNEL") &&
                        (n_cols + 1) * (uint64_t)kPredPitch * sizeof(float) <= 40ull * 1024;

@@ -9,7 +9,7 @@ extern "C" hipError_t hipExtModuleLaunchKernel(hipFunction_t f, uint32_t globalW
                                                hipEvent_t startEvent, hipEvent_t stopEvent, uint32_t flags);
 
 #include <dlfcn.h>
-#include <omp.h>
+#include <sched.h>
 #include <algorithm>
 #include <cstdlib>
 
@@ -177,22 +177,6 @@ void Device::reset_stats() {
     stats_.clear();
 }
 
-// Pageable host bytes into pinned memory with the host's threads (one
-// thread's memcpy reaches a fraction of the link's rate). The thread count
-// is the processors', whatever the process last set for its own parallel
-// regions.
-static void copy_threads(void *dst, const void *src, uint64_t bytes) {
-    constexpr uint64_t kPiece = 256ull << 10;
-    const int64_t pieces = (int64_t)((bytes + kPiece - 1) / kPiece);
-    const int threads = std::max(1, std::min(32, omp_get_num_procs()));
-#pragma omp parallel for schedule(static) num_threads(threads)
-    for (int64_t i = 0; i < pieces; i++) {
-        const uint64_t off = (uint64_t)i * kPiece;
-        std::memcpy(static_cast<char *>(dst) + off, static_cast<const char *>(src) + off,
-                    std::min<uint64_t>(kPiece, bytes - off));
-    }
-}
-
 void Device::host_rows(const float *x, uint64_t n, uint64_t n_cols, uint64_t chunk_rows,
                        const std::function<void(const float *, uint64_t, uint64_t)> &fn) {
     if (n == 0) return;
@@ -200,6 +184,11 @@ void Device::host_rows(const float *x, uint64_t n, uint64_t n_cols, uint64_t chu
     std::lock_guard<std::mutex> lock(pipe_mu_);
     const uint64_t row_bytes = n_cols * sizeof(float);
     const uint64_t bytes = std::min(chunk_rows, n) * row_bytes;
+    if (!pipe_threads_) {  // eight threads, the caller's among them, reach the link's rate
+        cpu_set_t cpus;
+        const int n = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+        pipe_threads_ = std::make_unique<CopyPool>((unsigned)std::min(n, 8) - 1u);
+    }
     if (!pipe_copy_) {
         HBR_HIP(hipStreamCreateWithFlags(&pipe_copy_, hipStreamNonBlocking));
         for (int b = 0; b < 2; b++) {
@@ -232,7 +221,7 @@ void Device::host_rows(const float *x, uint64_t n, uint64_t n_cols, uint64_t chu
         // the copy two chunks back has read this staging buffer, and the
         // work last queued on this device buffer has read it
         if (c >= 2) HBR_HIP(hipEventSynchronize(pipe_copied_[b]));
-        copy_threads(pipe_stage_[b], x + r0 * n_cols, rows * row_bytes);
+        pipe_threads_->copy(pipe_stage_[b], x + r0 * n_cols, rows * row_bytes);
         // (an earlier call's last chunks count: their work may still run)
         if (pipe_used_set_[b]) HBR_HIP(hipStreamWaitEvent(pipe_copy_, pipe_used_[b], 0));
         HBR_HIP(hipMemcpyAsync(pipe_rows_[b], pipe_stage_[b], rows * row_bytes, hipMemcpyHostToDevice, pipe_copy_));

@@ -7,10 +7,13 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include "copy_pool.h"
+
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -109,6 +112,7 @@ private:
     std::unordered_map<std::string, KernelStat> stats_;
     // host_rows' staging
     std::mutex pipe_mu_;
+    std::unique_ptr<CopyPool> pipe_threads_;
     hipStream_t pipe_copy_ = nullptr;
     hipEvent_t pipe_copied_[2] = {nullptr, nullptr};  // a chunk's copy has read its staging buffer
     hipEvent_t pipe_used_[2] = {nullptr, nullptr};    // the queued work has read a device buffer
