@@ -87,6 +87,7 @@ Device::~Device() {
 void Device::activate() const { HBR_HIP(hipSetDevice(ordinal_)); }
 
 hipFunction_t Device::function(const char *kernel) {
+    std::lock_guard<std::mutex> lock(functions_mu_);  // engines and forests of several threads launch here
     auto it = functions_.find(kernel);
     if (it != functions_.end()) return it->second;
     hipFunction_t f;

@@ -98,6 +98,7 @@ private:
     int cu_count_ = 0;
     hipStream_t stream_ = nullptr;
     hipModule_t module_ = nullptr;
+    std::mutex functions_mu_;
     std::unordered_map<std::string, hipFunction_t> functions_;
     uint32_t profile_every_ = 0;
     uint64_t profile_seen_ = 0;

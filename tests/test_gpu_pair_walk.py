@@ -66,3 +66,31 @@ def test_host_rows_of_every_size_equal_device_rows(n, outputs):
     for _ in range(2):
         assert np.array_equal(forest.predict_margin(x).view(np.uint32), want.view(np.uint32))
         assert np.array_equal(forest.predict_margin(x, init_margins=init).view(np.uint32), want.view(np.uint32))
+
+
+def test_forests_in_several_threads_share_the_device():
+    """Each its own forest, sizes that are read in place, copied and staged in
+    turn: every thread gets what it gets alone."""
+    import threading
+
+    rng = np.random.default_rng(3)
+    k, f = 4, 30
+    forests = [hb.Forest(_forest(rng, 20 + 9 * i, 4, f, 1 + i % 2), 1 + i % 2) for i in range(k)]
+    rows = [[rng.standard_normal((n, f), dtype=np.float32) for n in (1, 900, 3_000, 12_000, 60_000)] for _ in range(k)]
+    alone = [[forests[i].predict_margin(x) for x in rows[i]] for i in range(k)]
+    wrong, gate = [], threading.Barrier(k)
+
+    def work(i):
+        gate.wait()
+        for turn in range(12):
+            for j in range(len(rows[i])):
+                at = (j + i + turn) % len(rows[i])
+                if not np.array_equal(forests[i].predict_margin(rows[i][at]), alone[i][at]):
+                    wrong.append((i, at, turn))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(k)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
