@@ -467,12 +467,14 @@ void Forest::predict_device(const float *x, uint64_t n, uint64_t n_cols, float m
 // - a few (256 KiB): copied into pinned memory, which the pair walk reads and
 //   writes in place: one launch and one wait instead of a copy each way
 //   around it (32 rows of 28 features: 34.1 -> 22.3 us a call);
-// - up to 1 MiB, or another walk: one copy each way;
+// - up to 8 MiB, or another walk: one copy each way (2.4 MB of 30 features
+//   0.132 ms, in chunks 0.150; 8 MB 0.30 and 0.28);
 // - more: in chunks, each staged by the host's threads and copied while the
-//   walk runs on the one before (Device::host_rows); small enough that the
-//   first chunk's copy is little of the whole (500,000 x 30: 2,356 -> 1,450 us)
-//   and the device's staging, which stays, little memory (1.6 GB: 31.6 ms in
-//   chunks of 16 MiB, 34.3 in chunks of 128).
+//   walk runs on the one before (Device::host_rows); large enough (2 MiB) that
+//   the waits between them are little (12 MB: 0.387 ms, in chunks of 1 MiB
+//   0.447), small enough that the first chunk's copy is (500,000 x 30: 2,356 ->
+//   1,450 us) and that the device's staging, which stays, takes little memory
+//   (1.6 GB: 31.6 ms in chunks of 16 MiB, 34.3 in chunks of 128).
 // The other buffers stay with the forest up to kKeepBytes.
 void Forest::predict_host(const float *x, uint64_t n, uint64_t n_cols, float missing, float *out,
                           const float *init) {
@@ -480,7 +482,7 @@ void Forest::predict_host(const float *x, uint64_t n, uint64_t n_cols, float mis
     const uint64_t k = n_outputs_;
     const uint64_t row_bytes = n_cols * sizeof(float), out_bytes = n * k * sizeof(float);
     hipStream_t s = dev_.stream();
-    constexpr uint64_t kDirectRows = Device::kDirectBytes / 2, kPipeBytes = 1ull << 20, kChunkBytes = 16ull << 20;
+    constexpr uint64_t kDirectRows = Device::kDirectBytes / 2, kPipeBytes = 8ull << 20, kChunkBytes = 16ull << 20;
     constexpr uint64_t kKeepBytes = 64ull << 20;
     const bool pairs = n_trees_ && pairs_ok_ && !std::getenv("HBROCM_PRED_KERNEL") &&
                        (n_cols + 1) * (uint64_t)kPredPitch * sizeof(float) <= 40ull * 1024;
@@ -509,7 +511,7 @@ void Forest::predict_host(const float *x, uint64_t n, uint64_t n_cols, float mis
         host_x_.upload(x, n * n_cols, s);
         predict_device(host_x_.get(), n, n_cols, missing, host_out_.get(), nullptr, init_dev);
     } else {
-        const uint64_t bytes = std::min(kChunkBytes, std::max(kPipeBytes, n * row_bytes / 8));
+        const uint64_t bytes = std::min(kChunkBytes, std::max(kPipeBytes / 4, n * row_bytes / 8));
         const uint64_t chunk_rows = std::max<uint64_t>(64, bytes / row_bytes / 64 * 64);
         dev_.host_rows(x, n, n_cols, chunk_rows, [&](const float *rows_dev, uint64_t r0, uint64_t rows) {
             predict_device(rows_dev, rows, n_cols, missing, host_out_.get() + r0 * k, nullptr,

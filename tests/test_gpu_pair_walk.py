@@ -49,8 +49,8 @@ def test_shared_blocks_equal_the_mirror_walk(monkeypatch, n, trees, depth, f, ou
 
 
 
-# host rows read in place (up to 256 KiB), in one copy (up to 1 MiB), in chunks
-@pytest.mark.parametrize("n", [1, 700, 1_250, 2_180, 2_200, 8_700, 8_800, 20_011])
+# host rows read in place (up to 256 KiB), in one copy (up to 8 MiB), in chunks
+@pytest.mark.parametrize("n", [1, 700, 1_250, 2_180, 2_200, 8_700, 8_800, 20_011, 69_905, 69_906, 150_001])
 @pytest.mark.parametrize("outputs", [1, 3])
 def test_host_rows_of_every_size_equal_device_rows(n, outputs):
     rng = np.random.default_rng(n + outputs)
@@ -76,7 +76,7 @@ def test_forests_in_several_threads_share_the_device():
     rng = np.random.default_rng(3)
     k, f = 4, 30
     forests = [hb.Forest(_forest(rng, 20 + 9 * i, 4, f, 1 + i % 2), 1 + i % 2) for i in range(k)]
-    rows = [[rng.standard_normal((n, f), dtype=np.float32) for n in (1, 900, 3_000, 12_000, 60_000)] for _ in range(k)]
+    rows = [[rng.standard_normal((n, f), dtype=np.float32) for n in (1, 900, 3_000, 12_000, 75_000)] for _ in range(k)]
     alone = [[forests[i].predict_margin(x) for x in rows[i]] for i in range(k)]
     wrong, gate = [], threading.Barrier(k)
 
