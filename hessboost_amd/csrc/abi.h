@@ -500,7 +500,7 @@ struct ReduceArgs {
     uint32_t total_bins;
     uint32_t groups;
     uint32_t fg;
-    const GrowCounts *grow;     // hbr_reduce_scan: nodes = its n_splits (the grid covers the most)
+    const GrowCounts *grow;     // non-null: nodes = its n_splits (the grid covers the most)
     uint32_t group_bins;        // bins per feature in a partial: 256 (u8 rows) or kWideLdsBins / fg
     uint32_t quarters;          // workgroups per feature: group_bins / 64
 };

@@ -204,8 +204,9 @@ public:
     // ---- depthwise growth on the device ----------------------------------------
     // A whole depthwise tree decided level by level on the device from the
     // staged gradients and read back with one synchronisation: the nodes in
-    // tree order. Needs a dense u8 index (the depth limit's rows are routed
-    // by the walk, not partitioned) and max_depth in [1, kMaxDeviceDepth].
+    // tree order. Needs rows of u8 bins, or of u16 bins and their columns (the
+    // depth limit's rows are routed by the walk, not partitioned), numeric
+    // features and max_depth in [1, kMaxDeviceDepth].
     static constexpr uint32_t kMaxDeviceDepth = 13;
     bool can_grow_device(uint64_t max_depth, uint32_t n_trees = 1) const;
     // false when a gradient is not finite

@@ -71,15 +71,17 @@ def _fit(monkeypatch, x, y, params, device):
 # few bins a feature beside one of many (a tile's sums take 128 KiB for every
 # feature then), and many features of two bins (128 KiB for every 32): a deep
 # level's nodes may not each take that much
-@pytest.mark.parametrize("f,depth,widest,max_bin", [(300, 10, 5_000, 5_000), (2_000, 11, 2, 256), (2_000, 12, 2, 256),
-                                                    (33, 10, 2, 256)])
-def test_deep_levels_of_few_bins_take_little_memory(monkeypatch, f, depth, widest, max_bin):
+@pytest.mark.parametrize("f,depth,widest,max_bin,nan", [
+    (300, 10, 5_000, 5_000, 0.0), (2_000, 11, 2, 256, 0.0), (2_000, 12, 2, 256, 0.0), (33, 10, 2, 256, 0.0),
+    (200, 10, 2, 256, 0.1)])
+def test_deep_levels_of_few_bins_take_little_memory(monkeypatch, f, depth, widest, max_bin, nan):
     rng = np.random.default_rng(f + depth)
     n = 6_000
     x = rng.integers(0, 2, (n, f)).astype(np.float32)
     if widest > 2:
         x[:, 5] = rng.permutation(n).astype(np.float32)
     y = (x[:, :12] @ rng.standard_normal(12) + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    x[rng.random(x.shape) < nan] = np.nan
     params = {"objective": "reg:squarederror", "max_depth": depth, "eta": 0.3, "max_bin": max_bin}
     trees, margins, used = _fit(monkeypatch, x, y, params, True)
     want, want_margins, _ = _fit(monkeypatch, x, y, params, False)
