@@ -1335,8 +1335,9 @@ bool Engine::scan_reduces(uint32_t n, size_t shared, size_t per_node) const {
 // Histograms of a batch of nodes into their slots: the plan kernel cuts the
 // nodes' rows into tiles (about `per_cu` resident workgroups per CU over the
 // launch), then one workgroup per (tile, feature group). Dense u8 tiles
-// write their sums with plain stores (the reduce kernel adds up nodes of
-// several tiles); CSR tiles add into slots zeroed first.
+// and CSR ones write their sums with plain stores, to the slot or, for nodes of
+// several tiles, to partials that the reduce kernel (or the level's search)
+// adds up.
 void Engine::launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vector<HistNode> *host_nodes,
                          const PartSplit *splits_dev, const PartOut *part_out_dev, const uint32_t *rows0,
                          const GrowCounts *grow) {

@@ -376,8 +376,7 @@ private:
     bool identity_rows0_ = false;
     bool rows0_written_ = false;
     void write_identity_rows();  // buffer 0 := 0..n-1, once per tree, when a row list is read
-    // `n` nodes (the most a device-grown level can hold, with `grow`);
-    // host_nodes: their slots are zeroed first (CSR)
+    // `n` nodes (the most a device-grown level can hold, with `grow`)
     void launch_hist(const HistNode *nodes_dev, uint32_t n, const std::vector<HistNode> *host_nodes,
                      const PartSplit *splits_dev, const PartOut *part_out_dev, const uint32_t *rows0 = nullptr,
                      const GrowCounts *grow = nullptr);

@@ -13,8 +13,8 @@
 // a workgroup takes one tile and one group of FG features, accumulates into
 // LDS with 64-bit integer atomics, then writes its sub-histogram with plain
 // stores: straight into the node's slot when the node is one tile, else to
-// a partial that hbr_hist_reduce sums. No device-scope atomics.
-// Sparse (CSR) indexes add each stored entry straight to the slot.
+// a partial that hbr_hist_reduce (or hbr_reduce_scan) sums. No device-scope
+// atomics. Sparse (CSR) indexes do the same by ranges of global bins.
 #include "common.h"
 
 namespace hbr {
