@@ -186,28 +186,34 @@ constexpr uint32_t kGradRows = 2;
 extern "C" __global__ __launch_bounds__(1024) void hbr_gradients(GradArgs a) {
     uint32_t mg = 0, mh = 0, bad = 0;
     const uint32_t stride = gridDim.x * blockDim.x;
-    const uint64_t end = ((uint64_t)a.n + kWave - 1) / kWave * kWave;  // whole waves stay in the loop
-    // (64-bit places: a step past the last row may leave 32 bits)
-    for (uint64_t i0 = blockIdx.x * blockDim.x + threadIdx.x; i0 < end; i0 += kGradRows * stride) {
+    // whole waves stay in the loop; `room`: places after i0 up to the last
+    // wave's end (a step past it may leave 32 bits, so none is computed)
+    const uint32_t last = (a.n - 1u) | (kWave - 1u);
+    uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x;
+    bool more = a.n && i0 <= last;
+    while (more) {
+        const uint32_t room = last - i0;
         float m[kGradRows], y[kGradRows], w[kGradRows];
 #pragma unroll
         for (uint32_t k = 0; k < kGradRows; k++) {
-            const uint64_t i = i0 + k * stride;
-            const bool active = i < a.n;
+            const uint32_t i = i0 + k * stride;
+            const bool active = k * stride <= room && i < a.n;
             m[k] = active ? a.margins[i] : 0.0f;
             y[k] = active ? a.labels[i] : 0.0f;
             w[k] = active && a.weights ? a.weights[i] : 1.0f;
         }
 #pragma unroll
         for (uint32_t k = 0; k < kGradRows; k++) {
-            if (i0 + k * stride >= end) break;  // whole waves
-            const uint32_t i = (uint32_t)(i0 + k * stride);
-            const bool active = i0 + k * stride < a.n;
+            if (k * stride > room) break;  // whole waves
+            const uint32_t i = i0 + k * stride;
+            const bool active = i < a.n;
             uint32_t word = 0;
             row_gradient_yw<false>(a, i, i, active, m[k], y[k], w[k], mg, mh, bad, &word);
             if (a.pair_rows && active)  // uniform flag; one word in the row's padding
                 *reinterpret_cast<uint32_t *>(a.pair_rows + (size_t)i * a.pair_stride + a.pair_byte) = word;
         }
+        more = kGradRows * stride <= room;
+        i0 += kGradRows * stride;
     }
     fold_block(a.scale, mg, mh, bad);
 }
